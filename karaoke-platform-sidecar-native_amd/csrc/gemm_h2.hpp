@@ -31,7 +31,10 @@
 // (|gelu(g)| <= |g|), a tanh output 1.  The bound only has to hold: a loose
 // one costs precision only for elements more than 2^17 below it.
 //
-// Operands and pipeline as gemm_split.hpp (256x128 block, 8 waves of 32x128,
+// Block tiles (H2Tile) of 256x128 and 128x128 (waves of 32x128) where a launch
+// fills the chip's 256 CUs several times over, of 64x128 and 64x64 where it
+// does not (the launcher's rule says which; all give the same bits).
+// Operands and pipeline as gemm_split.hpp (for 256x128: 8 waves of 32x128,
 // K chunks of 16 in a global->LDS DMA ring, A fp32 in LDS split by each wave
 // in registers, or h2 rows read as they are): W's pieces are two fp16 planes
 // per tile-major block (8 KB per 128 rows x 16 k, the same row/slot
@@ -76,7 +79,7 @@ struct GemmDescH2 {
     int rope_period, rope_len;
 };
 
-// The fused projection's k or v column tile (32 x 128 per wave, n0 inside
+// The fused projection's k or v column tile (32 x 32 NJ per wave, n0 inside
 // [kv_inner, 3 kv_inner)) written as fp16 pieces instead of fp32: the head's
 // 64 columns of a row occupy its 256 bytes of the region -- 64 h halves, then
 // 64 m halves, dim order -- where h + m is the value y scaled by 2^ek (2^ev),
@@ -89,8 +92,9 @@ struct GemmDescH2 {
 // the bias in one fused multiply-add.
 // tv: the rotary table entry (cos, sin) of frame f0 (lanes 0-31) or f1
 // (lanes 32-63) and pair lane % 32, loaded before the K loop (k tiles only).
+template <int NJ>
 VH_DEVICE void kv_pieces_epilogue(const GemmDescH2 &d, int row0, int n0, int li, int lh, float2 tv,
-                                  const floatx16 (&acc)[1][4], floatx16 rs, floatx4 bpre) {
+                                  const floatx16 (&acc)[1][NJ], floatx16 rs, floatx4 bpre) {
     const bool is_k = n0 < 2 * d.kv_inner;
     const int region = is_k ? d.kv_inner : 2 * d.kv_inner;  // first column of the k (v) region
     const int B = d.rope_period;
@@ -108,7 +112,7 @@ VH_DEVICE void kv_pieces_epilogue(const GemmDescH2 &d, int row0, int n0, int li,
         constexpr bool IS_K = decltype(k_c)::value, FULL = decltype(full_c)::value;
         constexpr bool SPLIT = decltype(split_c)::value;
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
+        for (int j = 0; j < NJ; j++) {
             // one column tile at a time: nothing of the next is hoisted into
             // this one (the registers the K loop needs bound the epilogue's)
             __builtin_amdgcn_sched_barrier(0);
@@ -195,12 +199,31 @@ struct H2Bound {
     float value;
 };
 
+// A workgroup's tile: WR x WC waves of 32 rows x 32 NJ_ columns; a ring of
+// RING_ stages in LDS, each KS_ chunks of 16 of K, RING_ - 1 of them in flight
+// while one is multiplied; OCC_ waves per SIMD the register count must allow.
+template <int WR, int WC_, int NJ_, int KS_, int RING_, int OCC_>
+struct H2Tile {
+    static constexpr int WC = WC_, NJ = NJ_, KS = KS_, RING = RING_, OCC = OCC_;
+    static constexpr int WAVES = WR * WC, THREADS = 64 * WAVES;
+    static constexpr int BM = 32 * WR, BN = 32 * NJ * WC;
+    static_assert(BN <= GS_BN && GS_BN % BN == 0, "a tile's columns lie in one 128-row tile of the pieces");
+};
+using H2Tile256 = H2Tile<8, 1, 4, 1, 3, 2>;  // 256 x 128, 72 KB LDS: two workgroups per CU
+using H2Tile128 = H2Tile<4, 1, 4, 1, 3, 3>;  // 128 x 128, 48 KB: three
+// The small tiles take K 32 at a time (half the barriers: at one wave of work
+// per SIMD between them, they and the LDS latency are the time), which leaves
+// room for one stage in flight (a third stage, fewer workgroups per CU: +3-10%).
+using H2Tile64 = H2Tile<2, 2, 2, 2, 2, 3>;   // 64 x 128, 48 KB: three
+using H2Tile64n = H2Tile<2, 2, 1, 2, 2, 4>;  // 64 x 64, 32 KB: five
+
 constexpr int H2_HEADER = 256;                // bytes before the planes: float max|W|
 constexpr int H2_WBLOCK = 2 * GS_BN * GS_BK;  // fp16 per (row tile, K chunk) block of W pieces
 
 // A_H2: A arrives as h2 rows (h2.hpp) scaled by 2^h2_exponent(a_bound) -- its
 // producer split it -- and the K loop only reads the pieces.
-// RING: K chunks held in LDS, RING - 1 of them in flight while one is multiplied.
+// T: the block tile (H2Tile).  Every tile forms each output by the same
+// products in the same order: the results are the same bits.
 // NORM (fp32 A): the GEMM of an RMSNorm of A's rows, W holding the norm's gain
 // folded in (W[n][k] gamma[k]): each accumulator row is multiplied by its row's
 // sqrt(K) / sqrt(sum_k A^2 + 1e-12) (the RMSNorm kernels' expression), the
@@ -211,27 +234,35 @@ constexpr int H2_WBLOCK = 2 * GS_BN * GS_BK;  // fp16 per (row tile, K chunk) bl
 // KVS: the k and v columns scaled (GemmDescH2::kv_inner), compiled only into
 // the fused projection's instantiations, and with kv_pieces written as their
 // fp16 pieces (k rotated).
-template <int EPI, bool A_H2, int RING = 3, bool NORM = false, bool KVS = false>
+template <int EPI, bool A_H2, class T, bool NORM = false, bool KVS = false>
 __device__ __forceinline__ void gemm_h2_body(const GemmDescH2 &d, float a_bound, int tile) {
     static_assert(!(NORM && A_H2), "the row norm needs the fp32 rows");
-    constexpr int A_BYTES = GS_BM * GS_BK * 4;  // 16 KB: fp32 rows of 64 B
-    constexpr int P_BYTES = GS_BN * GS_BK * 2;  // 4 KB per W plane: fp16 rows of 32 B
-    constexpr int STAGE_BYTES = A_BYTES + 2 * P_BYTES;
+    static_assert(EPI != EPI_GEGLU || T::NJ % 2 == 0, "a wave holds the value and the gate columns");
+    constexpr int NJW = T::NJ, RING = T::RING, KS = T::KS;
+    constexpr int A_BYTES = T::BM * GS_BK * 4;  // fp32 rows of 64 B
+    constexpr int P_BYTES = T::BN * GS_BK * 2;  // per W plane: fp16 rows of 32 B
+    constexpr int SUB_BYTES = A_BYTES + 2 * P_BYTES;
+    constexpr int STAGE_BYTES = KS * SUB_BYTES;
+    // 1 KB loads of A and W per wave and chunk
+    constexpr int UA = T::BM / 16 / T::WAVES, UW = T::BN / 16 / T::WAVES;
+    static_assert(UA * T::WAVES * 16 == T::BM && UW * T::WAVES * 16 == T::BN, "whole 1 KB loads per wave");
+    constexpr int LOADS = KS * (UA + UW);  // per wave and stage
     __shared__ __attribute__((aligned(1024))) unsigned char ring[RING * STAGE_BYTES];
 
-    const int tiles_n = (d.N + GS_BN - 1) / GS_BN;
-    const int tiles_m = (d.M + GS_BM - 1) / GS_BM;
+    const int tiles_n = (d.N + T::BN - 1) / T::BN;
+    const int tiles_m = (d.M + T::BM - 1) / T::BM;
     if (d.zero_slot && tile == 0 && threadIdx.x == 0) *d.zero_slot = 0.0f;
     if (tile >= tiles_m * tiles_n) return;
     // column-fastest order within groups of row tiles (see gemm.hpp)
-    // groups of 4 row tiles for the wide GEMMs (measured against 1, 2, 8, 16:
-    // best by 0.3-1.3% on N = 1568 and 3072), one for N = 384
-    const int gsz = d.N >= 1024 ? 4 : 1;
+    // groups of 1024 rows for the wide GEMMs (256-row tiles: 4 measured
+    // against 1, 2, 8, 16, best by 0.3-1.3% on N = 1568 and 3072), one row
+    // tile for N = 384
+    const int gsz = d.N >= 1024 ? 1024 / T::BM : 1;
     const int group = tile / (gsz * tiles_n);
     const int in_group = tile % (gsz * tiles_n);
     const int group_rows = min(gsz, tiles_m - group * gsz);
-    const int m0 = (group * gsz + in_group % group_rows) * GS_BM;
-    const int n0 = (in_group / group_rows) * GS_BN;
+    const int m0 = (group * gsz + in_group % group_rows) * T::BM;
+    const int n0 = (in_group / group_rows) * T::BN;
 
     const int ea = h2_exponent(a_bound);
     const int ew = h2_exponent(*static_cast<const float *>(d.W));
@@ -240,6 +271,8 @@ __device__ __forceinline__ void gemm_h2_body(const GemmDescH2 &d, float a_bound,
     const int tid = (int)threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 31, lh = lane >> 5;
+    const int wr = wave / T::WC, wc = wave % T::WC;  // the wave's 32 rows and 32 NJ columns
+    const int row0 = m0 + 32 * wr, col0 = n0 + 32 * NJW * wc;
     const uint32_t ring_base = (uint32_t)(uintptr_t)ring;
     auto swz_a = [](int r) { return (r >> 2) & 3; };
     auto swz_w = [](int r) { return (r >> 3) & 1; };
@@ -247,10 +280,10 @@ __device__ __forceinline__ void gemm_h2_body(const GemmDescH2 &d, float a_bound,
     // the bias of the lane's column in each 32-column tile (0 past N), loaded
     // before the K loop so that its latency is spent there, not in the
     // epilogue
-    float bpre[4];
+    float bpre[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int col = n0 + 32 * j + li;
+    for (int j = 0; j < NJW; j++) {
+        const int col = col0 + 32 * j + li;
         bpre[j] = d.bias && col < d.N ? d.bias[col] : 0.0f;
     }
     // each 32-column tile's extra power of two: ek for k columns, ev for v
@@ -260,138 +293,151 @@ __device__ __forceinline__ void gemm_h2_body(const GemmDescH2 &d, float a_bound,
         int ek, eq, ev;
         att_h2_exponents(*d.kv_bound, 1.0f, ek, eq, ev);
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int c = n0 + 32 * j;
+        for (int j = 0; j < NJW; j++) {
+            const int c = col0 + 32 * j;
             ekv[j] = c < d.kv_inner ? 0 : c < 2 * d.kv_inner ? ek : c < 3 * d.kv_inner ? ev : 0;
         }
     }
 
-    // A: 16 loads of 1 KB (16 rows each), wave w loads blocks w and w+8 from
-    // the tile's first row (scalar base) plus its lane offset (below 2^32:
-    // 256 rows of lda <= 2^21 floats).  W: the 8 1 KB blocks of the chunk's
-    // tile-major image, wave w the w-th.
+    // A: 1 KB loads of 16 rows each, wave w loads blocks w, w + WAVES, ...
+    // from the tile's first row (scalar base) plus its lane offset (below
+    // 2^32: at most 256 rows of lda <= 2^21 floats).  W: the tile's rows of
+    // each plane of the chunk's 128-row tile-major image, consecutive there:
+    // blocks w, w + WAVES, ... of 1 KB, the h plane's first.
     const float *a_base = d.A + (size_t)m0 * d.lda;
-    uint32_t a_voff[2];
+    uint32_t a_voff[UA];
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int r = 16 * (wave + 8 * j) + (lane >> 2);
+    for (int j = 0; j < UA; j++) {
+        const int r = 16 * (wave + T::WAVES * j) + (lane >> 2);
         a_voff[j] = (uint32_t)(min(m0 + r, d.M - 1) - m0) * (uint32_t)d.lda * 4u + 16u * ((lane & 3) ^ swz_a(r));
     }
     const _Float16 *w_base = reinterpret_cast<const _Float16 *>(static_cast<const char *>(d.W) + H2_HEADER) +
-                             (size_t)(n0 / GS_BN) * (d.K / GS_BK) * H2_WBLOCK;
+                             (size_t)(n0 / GS_BN) * (d.K / GS_BK) * H2_WBLOCK + (n0 % GS_BN) * GS_BK;
     const uint32_t w_voff = 16 * lane;
-    auto issue = [&](int kt) {
-        const uint32_t sb = ring_base + (kt % RING) * STAGE_BYTES;
-        const float *ab = a_base + kt * GS_BK;
-        lds_dma16s(a_voff[0], ab, sb + wave * 1024);
-        lds_dma16s(a_voff[1], ab, sb + (wave + 8) * 1024);
-        lds_dma16s(w_voff, w_base + (size_t)kt * H2_WBLOCK + wave * 512, sb + A_BYTES + wave * 1024);
+    auto issue = [&](int st) {
+#pragma unroll
+        for (int u = 0; u < KS; u++) {
+            const int kt = st * KS + u;
+            const uint32_t sb = ring_base + (st % RING) * STAGE_BYTES + u * SUB_BYTES;
+            const float *ab = a_base + kt * GS_BK;
+#pragma unroll
+            for (int j = 0; j < UA; j++) lds_dma16s(a_voff[j], ab, sb + (wave + T::WAVES * j) * 1024);
+#pragma unroll
+            for (int j = 0; j < UW; j++) {
+                const int i = wave + T::WAVES * j;
+                const int plane = i / (T::BN / 32), blk = i % (T::BN / 32);
+                lds_dma16s(w_voff, w_base + (size_t)kt * H2_WBLOCK + plane * (GS_BN * GS_BK) + blk * 512,
+                           sb + A_BYTES + i * 1024);
+            }
+        }
     };
 
-    floatx16 acc[1][4];
+    floatx16 acc[1][NJW];
 #pragma unroll
-    for (int j = 0; j < 4; j++)
+    for (int j = 0; j < NJW; j++)
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[0][j][r] = 0.0f;
 
     // k/v pieces: the rotary table entries the epilogue of a k tile needs,
     // loaded now so that their latency is spent in the K loop (two registers)
     float2 tv = make_float2(1.0f, 0.0f);
-    if constexpr (KVS && NORM && EPI == EPI_STORE) {
-        if (d.kv_pieces && n0 >= d.kv_inner && n0 < 2 * d.kv_inner) {
-            const int row0 = m0 + wave * 32;
+    if constexpr (KVS && EPI == EPI_STORE) {
+        if (d.kv_pieces && col0 >= d.kv_inner && col0 < 2 * d.kv_inner) {
             const int f0 = (row0 / d.rope_period) % d.rope_len;
             const int f = lane < 32 ? f0 : (f0 + 1 == d.rope_len ? 0 : f0 + 1);
             tv = *reinterpret_cast<const float2 *>(d.rope + 2 * (f * 32 + (lane & 31)));
         }
     }
-    const int nk = d.K / GS_BK;
-    float ss = 0.0f;  // NORM: sum of squares of this lane's half of row wave*32 + li
+    const int ns = d.K / (GS_BK * KS);  // stages (KS > 1: the launcher checked K)
+    float ss = 0.0f;  // NORM: sum of squares of this lane's half of row 32 wr + li
 #pragma unroll
     for (int i = 0; i < RING - 1; i++)
-        if (i < nk) issue(i);
-    if constexpr (RING > 2) {
-        if (nk > 1) wait_vmcnt<3 * (RING - 2)>();  // chunk 0 has landed
-        else wait_vmcnt<0>();
-    } else {
-        wait_vmcnt<0>();
-    }
+        if (i < ns) issue(i);
+    // stage 0 has landed once at most the stages issued after it are in flight
+    if (ns >= RING - 1) wait_vmcnt<LOADS *(RING - 2)>();
+    else wait_vmcnt<0>();
     __syncthreads();
     // NJ live 32-column accumulators, chosen once per tile (as gemm_split_body)
     auto k_loop = [&](auto nj_c) {
         constexpr int NJ = decltype(nj_c)::value;
-        for (int kt = 0; kt < nk; kt++) {
-            // chunk kt+RING-1 goes to the slot chunk kt-1 used: every wave
+        for (int st = 0; st < ns; st++) {
+            // stage st+RING-1 goes to the slot stage st-1 used: every wave
             // finished reading it before the barrier that ended the previous
             // iteration
-            if (kt + RING - 1 < nk) issue(kt + RING - 1);
-            const unsigned char *sbuf = ring + (kt % RING) * STAGE_BYTES;
-            const int r = wave * 32 + li;
-            const unsigned char *ar = sbuf + r * 64;
-            halfx8 ah, am;
-            if constexpr (A_H2) {
-                ah = *reinterpret_cast<const halfx8 *>(ar + 16 * (lh ^ swz_a(r)));
-                am = *reinterpret_cast<const halfx8 *>(ar + 16 * ((2 + lh) ^ swz_a(r)));
-            } else {
-                const floatx4 lo = *reinterpret_cast<const floatx4 *>(ar + 16 * (lh ^ swz_a(r)));
-                const floatx4 hi = *reinterpret_cast<const floatx4 *>(ar + 16 * ((2 + lh) ^ swz_a(r)));
-                split8_h2(lo, hi, a_scale, ah, am);
-                if constexpr (NORM) {
+            if (st + RING - 1 < ns) issue(st + RING - 1);
 #pragma unroll
-                    for (int e = 0; e < 4; e++) ss = fmaf(hi[e], hi[e], fmaf(lo[e], lo[e], ss));
+            for (int u = 0; u < KS; u++) {
+                const unsigned char *sbuf = ring + (st % RING) * STAGE_BYTES + u * SUB_BYTES;
+                const int r = wr * 32 + li;
+                const unsigned char *ar = sbuf + r * 64;
+                halfx8 ah, am;
+                if constexpr (A_H2) {
+                    ah = *reinterpret_cast<const halfx8 *>(ar + 16 * (lh ^ swz_a(r)));
+                    am = *reinterpret_cast<const halfx8 *>(ar + 16 * ((2 + lh) ^ swz_a(r)));
+                } else {
+                    const floatx4 lo = *reinterpret_cast<const floatx4 *>(ar + 16 * (lh ^ swz_a(r)));
+                    const floatx4 hi = *reinterpret_cast<const floatx4 *>(ar + 16 * ((2 + lh) ^ swz_a(r)));
+                    split8_h2(lo, hi, a_scale, ah, am);
+                    if constexpr (NORM) {
+#pragma unroll
+                        for (int e = 0; e < 4; e++) ss = fmaf(hi[e], hi[e], fmaf(lo[e], lo[e], ss));
+                    }
+                }
+                // W column tiles two at a time: their pieces, then (m,h) (h,m) (h,h)
+#pragma unroll
+                for (int jp = 0; jp < (NJ + 1) / 2; jp++) {
+                    constexpr int NJJ = NJ == 1 ? 1 : 2;
+                    halfx8 wh[NJJ], wm[NJJ];
+#pragma unroll
+                    for (int jj = 0; jj < NJJ; jj++) {
+                        const int rw = 32 * (NJW * wc + 2 * jp + jj) + li;
+                        const unsigned char *wp = sbuf + A_BYTES + rw * 32 + 16 * (lh ^ swz_w(rw));
+                        wh[jj] = *reinterpret_cast<const halfx8 *>(wp);
+                        wm[jj] = *reinterpret_cast<const halfx8 *>(wp + P_BYTES);
+                    }
+#pragma unroll
+                    for (int jj = 0; jj < NJJ; jj++)
+                        acc[0][2 * jp + jj] =
+                            __builtin_amdgcn_mfma_f32_32x32x16_f16(am, wh[jj], acc[0][2 * jp + jj], 0, 0, 0);
+#pragma unroll
+                    for (int jj = 0; jj < NJJ; jj++)
+                        acc[0][2 * jp + jj] =
+                            __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, wm[jj], acc[0][2 * jp + jj], 0, 0, 0);
+#pragma unroll
+                    for (int jj = 0; jj < NJJ; jj++)
+                        acc[0][2 * jp + jj] =
+                            __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, wh[jj], acc[0][2 * jp + jj], 0, 0, 0);
                 }
             }
-            // W column tiles two at a time: their pieces, then (m,h) (h,m) (h,h)
-#pragma unroll
-            for (int jp = 0; jp < (NJ + 1) / 2; jp++) {
-                constexpr int NJJ = NJ == 1 ? 1 : 2;
-                halfx8 wh[NJJ], wm[NJJ];
-#pragma unroll
-                for (int jj = 0; jj < NJJ; jj++) {
-                    const int rw = 32 * (2 * jp + jj) + li;
-                    const unsigned char *wp = sbuf + A_BYTES + rw * 32 + 16 * (lh ^ swz_w(rw));
-                    wh[jj] = *reinterpret_cast<const halfx8 *>(wp);
-                    wm[jj] = *reinterpret_cast<const halfx8 *>(wp + P_BYTES);
-                }
-#pragma unroll
-                for (int jj = 0; jj < NJJ; jj++)
-                    acc[0][2 * jp + jj] = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, wh[jj], acc[0][2 * jp + jj], 0, 0, 0);
-#pragma unroll
-                for (int jj = 0; jj < NJJ; jj++)
-                    acc[0][2 * jp + jj] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, wm[jj], acc[0][2 * jp + jj], 0, 0, 0);
-#pragma unroll
-                for (int jj = 0; jj < NJJ; jj++)
-                    acc[0][2 * jp + jj] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, wh[jj], acc[0][2 * jp + jj], 0, 0, 0);
-            }
-            // chunk kt+1 has landed (3 loads per wave and chunk; later chunks may fly)
-            if constexpr (RING > 2) {
-                if (kt + RING - 1 < nk) wait_vmcnt<3 * (RING - 2)>();
-                else wait_vmcnt<0>();
-            } else {
-                wait_vmcnt<0>();
-            }
+            // stage st+1 has landed (LOADS loads per wave and stage; later stages may fly)
+            if (st + RING - 1 < ns) wait_vmcnt<LOADS *(RING - 2)>();
+            else wait_vmcnt<0>();
             __syncthreads();
         }
     };
-    const int live = d.N - n0;
-    if (live > 64) k_loop(std::integral_constant<int, 4>());
-    else if (live > 32) k_loop(std::integral_constant<int, 2>());
-    else k_loop(std::integral_constant<int, 1>());
+    if constexpr (T::WC == 1 && NJW == 4) {
+        const int live = d.N - n0;
+        if (live > 64) k_loop(std::integral_constant<int, 4>());
+        else if (live > 32) k_loop(std::integral_constant<int, 2>());
+        else k_loop(std::integral_constant<int, 1>());
+    } else {
+        k_loop(std::integral_constant<int, NJW>());
+    }
     // both scales undone at once: acc 2^-(ea+ew) by one v_ldexp_f32 (exact, as
     // the two power-of-two multiplies it replaces were where their product
     // is a normal float, and correctly rounded where it is not)
     const int eu = -(ea + ew);
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
+    for (int j = 0; j < NJW; j++) {
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[0][j][r] = ldexpf(acc[0][j][r], eu + ekv[j]);
         bpre[j] = ldexpf(bpre[j], ekv[j]);  // (acc + b) 2^e exactly, with the row norm too
     }
     float rs[16];  // NORM: the scale of each accumulator row, applied with the bias
     if constexpr (NORM) {
-        // lanes li and li + 32 summed the two halves of row wave*32 + li;
+        // lanes li and li + 32 summed the two halves of row 32 wr + li;
         // register 4q + e of a lane holds row 8q + 4lh + e of the wave's 32
-        __shared__ float rscale[GS_THREADS / 64][32];
+        __shared__ float rscale[T::WAVES][32];
         const float tot = ss + __shfl_xor(ss, 32, 64);
         if (lh == 0) rscale[wave][li] = sqrtf((float)d.K) / sqrtf(tot + 1.0e-12f);
         __syncthreads();
@@ -402,8 +448,8 @@ __device__ __forceinline__ void gemm_h2_body(const GemmDescH2 &d, float a_bound,
             for (int e = 0; e < 4; e++) rs[4 * q + e] = r4[e];
         }
     }
-    if constexpr (KVS && NORM && EPI == EPI_STORE) {
-        if (d.kv_pieces && n0 >= d.kv_inner && n0 < 3 * d.kv_inner) {
+    if constexpr (KVS && EPI == EPI_STORE) {
+        if (d.kv_pieces && col0 >= d.kv_inner && col0 < 3 * d.kv_inner) {
             // the plain epilogue's value of each element (bias and row norm in
             // one fused multiply-add), formed in place first so the row
             // scales and biases are dead before the rotation and the split
@@ -411,37 +457,36 @@ __device__ __forceinline__ void gemm_h2_body(const GemmDescH2 &d, float a_bound,
             // keeps them in registers across the epilogue's variants
             floatx16 rsv;
 #pragma unroll
-            for (int r = 0; r < 16; r++) rsv[r] = rs[r];
-            kv_pieces_epilogue(d, m0 + wave * 32, n0, li, lh, tv, acc, rsv,
-                               floatx4{bpre[0], bpre[1], bpre[2], bpre[3]});
+            for (int r = 0; r < 16; r++) rsv[r] = NORM ? rs[r] : 1.0f;
+            kv_pieces_epilogue<NJW>(d, row0, col0, li, lh, tv, acc, rsv, floatx4{bpre[0], bpre[1], bpre[2], bpre[3]});
             return;
         }
     }
     GemmDescBF16 e{};
     e.bias = d.bias; e.C = d.C; e.M = d.M; e.N = d.N; e.K = d.K; e.ldc = d.ldc;
     float mx = 0.0f;
-    gemm_bf16_epilogue<EPI, float, 1, 4>(e, acc, m0 + wave * 32, n0, li, lh, &mx, bpre, NORM ? rs : nullptr);
+    gemm_bf16_epilogue<EPI, float, 1, NJW>(e, acc, row0, col0, li, lh, &mx, bpre, NORM ? rs : nullptr);
     if constexpr (EPI == EPI_RESIDUAL) {
         if (d.amax) {
             // one atomic per workgroup (one per wave, all on one address,
             // cost 17 us per launch of 4656 tiles); non-negative floats
             // order as their bit patterns
-            __shared__ float wmax[GS_THREADS / 64];
+            __shared__ float wmax[T::WAVES];
             mx = wave_max(mx);
             if (lane == 0) wmax[wave] = mx;
             __syncthreads();
             if (tid == 0) {
 #pragma unroll
-                for (int w = 1; w < GS_THREADS / 64; w++) mx = fmaxf(mx, wmax[w]);
+                for (int w = 1; w < T::WAVES; w++) mx = fmaxf(mx, wmax[w]);
                 atomicMax(reinterpret_cast<unsigned int *>(d.amax), __float_as_uint(mx));
             }
         }
     }
 }
 
-template <int EPI, bool A_H2, bool NORM = false, bool KVS = false>
-__global__ __launch_bounds__(GS_THREADS, 2) void gemm_h2_kernel(GemmDescH2 d, H2Bound b) {
-    gemm_h2_body<EPI, A_H2, 3, NORM, KVS>(d, b.ptr ? *b.ptr : b.value, xcd_swizzle((int)blockIdx.x, (int)gridDim.x));
+template <int EPI, bool A_H2, class T, bool NORM = false, bool KVS = false>
+__global__ __launch_bounds__(T::THREADS, T::OCC) void gemm_h2_kernel(GemmDescH2 d, H2Bound b) {
+    gemm_h2_body<EPI, A_H2, T, NORM, KVS>(d, b.ptr ? *b.ptr : b.value, xcd_swizzle((int)blockIdx.x, (int)gridDim.x));
 }
 
 // Ragged batch (the mask estimator's per-band linears): problem blockIdx.z,
@@ -451,9 +496,9 @@ struct GemmBatchH2 {
     H2Bound b;
 };
 
-template <int EPI>
-__global__ __launch_bounds__(GS_THREADS, 2) void gemm_h2_batched_kernel(GemmBatchH2 b) {
-    gemm_h2_body<EPI, false>(b.d[blockIdx.z], b.b.ptr ? *b.b.ptr : b.b.value, (int)blockIdx.x);
+template <int EPI, class T>
+__global__ __launch_bounds__(T::THREADS, T::OCC) void gemm_h2_batched_kernel(GemmBatchH2 b) {
+    gemm_h2_body<EPI, false, T>(b.d[blockIdx.z], b.b.ptr ? *b.b.ptr : b.b.value, (int)blockIdx.x);
 }
 
 // max |W| over W [N][ldw] (first K columns) into out[0]; one workgroup of

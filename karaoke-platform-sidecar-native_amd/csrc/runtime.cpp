@@ -409,23 +409,87 @@ static GemmDescH2 to_desc_h2(const GemmArgsH2 &g) {
     return d;
 }
 
-template <int EPI>
-static void launch_h2(hipStream_t s, const GemmDescH2 &d, const H2Bound &b, unsigned tiles, const GemmArgsH2 &g) {
+template <int EPI, class T>
+static void launch_h2(hipStream_t s, const GemmDescH2 &d, const H2Bound &b, const GemmArgsH2 &g) {
+    const dim3 grid((unsigned)(((g.M + T::BM - 1) / T::BM) * ((g.N + T::BN - 1) / T::BN))), block(T::THREADS);
     if constexpr (EPI == EPI_STORE || EPI == EPI_GELU || EPI == EPI_GEGLU) {
         if (g.row_norm) {  // gemm_h2_ok: fp32 A
             if constexpr (EPI == EPI_STORE) {
                 if (g.kv_inner) {  // the fused projection with k and v scaled
-                    hipLaunchKernelGGL((gemm_h2_kernel<EPI, false, true, true>), dim3(tiles), dim3(GS_THREADS), 0, s,
-                                       d, b);
+                    hipLaunchKernelGGL((gemm_h2_kernel<EPI, false, T, true, true>), grid, block, 0, s, d, b);
                     return;
                 }
             }
-            hipLaunchKernelGGL((gemm_h2_kernel<EPI, false, true>), dim3(tiles), dim3(GS_THREADS), 0, s, d, b);
+            hipLaunchKernelGGL((gemm_h2_kernel<EPI, false, T, true>), grid, block, 0, s, d, b);
             return;
         }
     }
-    if (g.a_h2) hipLaunchKernelGGL((gemm_h2_kernel<EPI, true>), dim3(tiles), dim3(GS_THREADS), 0, s, d, b);
-    else hipLaunchKernelGGL((gemm_h2_kernel<EPI, false>), dim3(tiles), dim3(GS_THREADS), 0, s, d, b);
+    if constexpr (EPI == EPI_STORE) {
+        if (g.kv_inner) {
+            hipLaunchKernelGGL((gemm_h2_kernel<EPI, true, T, false, true>), grid, block, 0, s, d, b);
+            return;
+        }
+    }
+    if (g.a_h2) hipLaunchKernelGGL((gemm_h2_kernel<EPI, true, T>), grid, block, 0, s, d, b);
+    else hipLaunchKernelGGL((gemm_h2_kernel<EPI, false, T>), grid, block, 0, s, d, b);
+}
+
+// CUs of the device (256 on an MI355X).
+static int device_cus() {
+    static int cus = 0;
+    if (cus == 0 && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, 0) != hipSuccess) cus = 256;
+    return cus;
+}
+
+// The block tile of a two-piece GEMM launch: the one of the least modelled
+// time, max(tiles on the fullest CU x a tile's share, a lone tile's time), in
+// units of a 128 x 128 block's time on 256 x 128 tiles on a full chip (38 us at
+// K = 1536).  A smaller tile costs more per element (W and A are copied and
+// read more often: 1, 1.08, 1.2, 1.47 measured on full chips) but divides a
+// launch into more even shares, and its lone time (2, 1.47, 0.95, 0.66; a
+// 256 x 128 tile alone on a CU takes as long as two) is shorter.  Measured with
+// the residual GEMM N = 384, K = 1536 (us on 256 x 128, 128 x 128, 64 x 128,
+// 64 x 64 tiles): M = 6262: 79, 61, 44, 42; 12524: 81, 67, 63, 70; 24862: 128,
+// 118, 108, 125; 49662: 228, 206, 228, 267; 77580: 291, 298, 333, 404; the
+// choice lies within 10% of the best of the four on both models' linears from
+// 1612 to 397296 rows.  Every tile gives the same bits.
+// tiles(bm, bn): workgroups of the launch.  The 64-row tiles take K in steps
+// of 32; a GELU-GLU wave needs 64 columns, which the 64 x 64 tile's has not.
+enum H2TileKind { H2_TILE_256, H2_TILE_128, H2_TILE_64, H2_TILE_64N };
+template <class Tiles>
+static H2TileKind h2_tile_pick(const Tiles &tiles, bool k32, bool geglu) {
+    struct Kind { int bm, bn; double share, lone; };
+    static const Kind kinds[4] = {{256, 128, 2.0, 2.0}, {128, 128, 1.08, 1.47}, {64, 128, 0.6, 0.95}, {64, 64, 0.3675, 0.66}};
+    const int n = !k32 ? 2 : geglu ? 3 : 4;
+    int best = 0;
+    double least = 0.0;
+    for (int i = 0; i < n; i++) {
+        const int64_t per_cu = (tiles(kinds[i].bm, kinds[i].bn) + device_cus() - 1) / device_cus();
+        const double t = std::max((double)per_cu * kinds[i].share, kinds[i].lone);
+        if (i == 0 || t < least) {
+            best = i;
+            least = t;
+        }
+    }
+    return (H2TileKind)best;
+}
+template <int EPI, class Go>
+static void with_h2_tile(H2TileKind kind, const Go &go) {
+    switch (kind) {
+        case H2_TILE_128: go(H2Tile128()); return;
+        case H2_TILE_64: go(H2Tile64()); return;
+        case H2_TILE_64N:
+            if constexpr (EPI != EPI_GEGLU) go(H2Tile64n());
+            return;
+        default: go(H2Tile256());
+    }
+}
+
+template <int EPI>
+static void launch_h2_any(hipStream_t s, const GemmDescH2 &d, const H2Bound &b, const GemmArgsH2 &g) {
+    auto tiles = [&](int bm, int bn) { return ((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn); };
+    with_h2_tile<EPI>(h2_tile_pick(tiles, g.K % 32 == 0, EPI == EPI_GEGLU),
+                      [&](auto tile) { launch_h2<EPI, decltype(tile)>(s, d, b, g); });
 }
 
 bool gemm_h2(hipStream_t s, const GemmArgsH2 &g, const OperandBound &bound, int epilogue, KernelTimer *t,
@@ -443,14 +507,13 @@ bool gemm_h2(hipStream_t s, const GemmArgsH2 &g, const OperandBound &bound, int 
     }
     const GemmDescH2 d = to_desc_h2(g);
     const H2Bound b{bound.dev, bound.value};
-    const unsigned tiles = (unsigned)(((g.M + GS_BM - 1) / GS_BM) * ((g.N + GS_BN - 1) / GS_BN));
     Scope sc(t, s, name);
     switch (epilogue) {
-        case EPI_STORE: launch_h2<EPI_STORE>(s, d, b, tiles, g); break;
-        case EPI_GELU: launch_h2<EPI_GELU>(s, d, b, tiles, g); break;
-        case EPI_TANH: launch_h2<EPI_TANH>(s, d, b, tiles, g); break;
-        case EPI_RESIDUAL: launch_h2<EPI_RESIDUAL>(s, d, b, tiles, g); break;
-        case EPI_GEGLU: launch_h2<EPI_GEGLU>(s, d, b, tiles, g); break;
+        case EPI_STORE: launch_h2_any<EPI_STORE>(s, d, b, g); break;
+        case EPI_GELU: launch_h2_any<EPI_GELU>(s, d, b, g); break;
+        case EPI_TANH: launch_h2_any<EPI_TANH>(s, d, b, g); break;
+        case EPI_RESIDUAL: launch_h2_any<EPI_RESIDUAL>(s, d, b, g); break;
+        case EPI_GEGLU: launch_h2_any<EPI_GEGLU>(s, d, b, g); break;
         default: set_error("unknown GEMM epilogue %d", epilogue); return false;
     }
     return sync_debug(s, "gemm_h2_kernel");
@@ -489,9 +552,35 @@ bool band_attention(hipStream_t s, const BandAttention &b, KernelTimer *t) {
     return sync_debug(s, "band_attention_fused_kernel");
 }
 
+// One launch: problem blockIdx.z, its grid that of the largest problem (the
+// workgroups past a problem's own tiles return at once and are not counted).
 template <int EPI>
-static void launch_h2_batched(hipStream_t s, const GemmBatchH2 &b, unsigned tiles, unsigned n) {
-    hipLaunchKernelGGL(gemm_h2_batched_kernel<EPI>, dim3(tiles, 1, n), dim3(GS_THREADS), 0, s, b);
+static void launch_h2_batched(hipStream_t s, const GemmBatchH2 &b, unsigned n) {
+    bool k32 = true;
+    for (unsigned i = 0; i < n; i++) k32 &= b.d[i].K % 32 == 0;
+    auto tiles_of = [&](unsigned i, int bm, int bn) {
+        return (int64_t)((b.d[i].M + bm - 1) / bm) * ((b.d[i].N + bn - 1) / bn);
+    };
+    auto tiles = [&](int bm, int bn) {
+        int64_t sum = 0;
+        for (unsigned i = 0; i < n; i++) sum += tiles_of(i, bm, bn);
+        return sum;
+    };
+    // Problems of few columns (N < 128) are bound by reading A, not by the
+    // products the rule counts: past one tile per CU of more than half-full
+    // 256-row tiles those stay (62 bands of 801 rows, K = 1536, N 16..1032: 157 us
+    // against 190, 189, 193 on the smaller ones; 64 of 87 rows: 43, 33, 29, 27).
+    int64_t rows = 0;
+    for (unsigned i = 0; i < n; i++) rows = std::max<int64_t>(rows, b.d[i].M);
+    const H2TileKind kind = rows > 128 && tiles(256, 128) > device_cus()
+                                ? H2_TILE_256
+                                : h2_tile_pick(tiles, k32, EPI == EPI_GEGLU);
+    with_h2_tile<EPI>(kind, [&](auto tile) {
+        using T = decltype(tile);
+        int64_t most = 0;
+        for (unsigned i = 0; i < n; i++) most = std::max(most, tiles_of(i, T::BM, T::BN));
+        hipLaunchKernelGGL((gemm_h2_batched_kernel<EPI, T>), dim3((unsigned)most, 1, n), dim3(T::THREADS), 0, s, b);
+    });
 }
 
 bool gemm_h2_batched(hipStream_t s, const std::vector<GemmArgsH2> &gs, const OperandBound &bound, int epilogue,
@@ -502,7 +591,6 @@ bool gemm_h2_batched(hipStream_t s, const std::vector<GemmArgsH2> &gs, const Ope
         GemmBatchH2 b;
         memset(&b, 0, sizeof(b));
         b.b = H2Bound{bound.dev, bound.value};
-        int64_t max_tiles = 0;
         for (size_t i = 0; i < count; i++) {
             const GemmArgsH2 &g = gs[first + i];
             if (!gemm_h2_ok(g, epilogue)) {
@@ -517,15 +605,14 @@ bool gemm_h2_batched(hipStream_t s, const std::vector<GemmArgsH2> &gs, const Ope
                 return false;
             }
             b.d[i] = to_desc_h2(g);
-            max_tiles = std::max(max_tiles, ((g.M + GS_BM - 1) / GS_BM) * ((g.N + GS_BN - 1) / GS_BN));
         }
-        const unsigned tiles = (unsigned)max_tiles, n = (unsigned)count;
+        const unsigned n = (unsigned)count;
         switch (epilogue) {
-            case EPI_STORE: launch_h2_batched<EPI_STORE>(s, b, tiles, n); break;
-            case EPI_GELU: launch_h2_batched<EPI_GELU>(s, b, tiles, n); break;
-            case EPI_TANH: launch_h2_batched<EPI_TANH>(s, b, tiles, n); break;
-            case EPI_RESIDUAL: launch_h2_batched<EPI_RESIDUAL>(s, b, tiles, n); break;
-            case EPI_GEGLU: launch_h2_batched<EPI_GEGLU>(s, b, tiles, n); break;
+            case EPI_STORE: launch_h2_batched<EPI_STORE>(s, b, n); break;
+            case EPI_GELU: launch_h2_batched<EPI_GELU>(s, b, n); break;
+            case EPI_TANH: launch_h2_batched<EPI_TANH>(s, b, n); break;
+            case EPI_RESIDUAL: launch_h2_batched<EPI_RESIDUAL>(s, b, n); break;
+            case EPI_GEGLU: launch_h2_batched<EPI_GEGLU>(s, b, n); break;
             default: set_error("unknown GEMM epilogue %d", epilogue); return false;
         }
         if (!sync_debug(s, "gemm_h2_batched_kernel")) return false;
@@ -836,10 +923,7 @@ bool attention(hipStream_t s, const void *qkv, int ld, void *out, int ld_out, co
     auto launch = [&](const AttnArgs &a) {
         if (lay.L <= 64 && !qkv_bf16) {
             // persistent: four workgroups per CU loop over the (sequence, head) tasks
-            static int cus = 0;
-            if (cus == 0 && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, 0) != hipSuccess)
-                cus = 256;
-            const unsigned grid = (unsigned)std::min<int64_t>((int64_t)lay.S * heads, 4 * (int64_t)cus);
+            const unsigned grid = (unsigned)std::min<int64_t>((int64_t)lay.S * heads, 4 * (int64_t)device_cus());
             if (a.bound) {  // fp16 two-piece products
                 if (out_bf16) hipLaunchKernelGGL((attention_short_h2_kernel<bf16>), dim3(grid), dim3(256), 0, s, a);
                 else if (kv_scaled)

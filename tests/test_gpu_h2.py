@@ -178,6 +178,27 @@ def test_gemm_h2_accuracy(ctx, rng, M, N, K, epi, has_bias):
         assert e_h2 <= 1.5 * e_fp32 + 1e-6
 
 
+@pytest.mark.parametrize("N,K,epi", [(384, 64, 3), (40, 96, 0), (1568, 32, 1), (192, 64, 4), (200, 48, 2)])
+def test_gemm_h2_tiles_same_bits(ctx, rng, N, K, epi):
+    """The launcher takes smaller block tiles for launches that do not fill the chip; every tile sums a product
+    in the same order, so the first rows of a large launch are those rows launched alone, bit for bit (edges of the
+    64, 128 and 256 row tiles, columns past 64 and 128, K with and without 32-wide steps)."""
+    big = 77600 if N >= 384 else 300000  # 256-row tiles
+    x = torch.randn(big, K, device="cuda:0", generator=torch.Generator("cuda:0").manual_seed(5))
+    planes = _pieces(ctx, (0.05 * rng.standard_normal((N, K))).astype(np.float32))
+    bias = to_dev(rng.standard_normal(N).astype(np.float32))
+    out = N // 2 if epi == native.EPI_GEGLU else N
+
+    def run(rows):
+        c = torch.ones(rows, out, device="cuda:0")
+        ctx.gemm_h2(x, planes, c, rows, N, K, bias=bias, epilogue=epi, a_bound=8.0)
+        return c
+
+    whole = run(big)
+    for rows in (1, 64, 65, 129, 257, 3000, 12525, 50001):
+        assert torch.equal(run(rows).view(torch.int32), whole[:rows].view(torch.int32)), rows
+
+
 def test_gemm_h2_geglu(ctx, rng):
     M, F, K = 333, 192, 384
     x = rng.standard_normal((M, K)).astype(np.float32)
