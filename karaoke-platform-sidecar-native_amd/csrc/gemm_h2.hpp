@@ -71,9 +71,11 @@ struct GemmDescH2 {
     int kv_inner;
     // kv_pieces (with kv_inner): k, rotated, and v are written as the fp16
     // pieces of those scaled values (kv_pieces_epilogue), the rotary position
-    // of row r being the frame (r / rope_period) % rope_len of rows ordered
-    // [chunk][frame][band] (rope_period bands per frame), its (cos, sin) at
-    // rope[(frame * 32 + pair) * 2]
+    // of row r being (r / rope_period) % rope_len -- rope_period >= 32: rows
+    // ordered [chunk][position][sequence], rope_period sequences per position
+    // (the time axis of [chunk][frame][band], the band axis of [band][frame]);
+    // 1: consecutive rows are consecutive positions, rope_len >= 32 of them --
+    // its (cos, sin) at rope[(position * 32 + pair) * 2]
     int kv_pieces;
     const float *rope;
     int rope_period, rope_len;
@@ -86,111 +88,134 @@ struct GemmDescH2 {
 // h = fp16(y), m = fp16(y - h) (exact difference): the pieces the two-piece
 // attention's staging forms, so the attention copies them into LDS as they
 // are.  k is rotated first (rope_own: each lane swaps its value with the
-// lane of the pair's other dimension), by the (cos, sin) of the row's frame;
-// a wave's 32 consecutive rows span at most two frames.  Each value is first
+// lane of the pair's other dimension), by the (cos, sin) of the row's
+// position; a wave's 32 consecutive rows span at most two positions, or
+// (rope_period 1) 32 of them, whose entries the lane loads four rows at a
+// time (cache hits; eight at a time took the kernel past 128 VGPRs).  Each value is first
 // formed as the plain epilogue forms it: acc times the row's norm scale plus
 // the bias in one fused multiply-add.
-// tv: the rotary table entry (cos, sin) of frame f0 (lanes 0-31) or f1
-// (lanes 32-63) and pair lane % 32, loaded before the K loop (k tiles only).
+// tv: the rotary table entry (cos, sin) of position f0 (lanes 0-31) or f1
+// (lanes 32-63) and pair lane % 32, loaded before the K loop (k tiles only,
+// rope_period > 1).
+// Stores.  A register quad holds four consecutive rows of the lane's column:
+// the four lanes of a quad swap halves (transpose4_f16) so that each holds
+// four consecutive columns of one row, and the wave lays a head's two column
+// tiles out in LDS (its own part of the ring, which the K loop no longer reads)
+// to leave as 16-byte stores of whole 256-byte rows.  Stored from registers the
+// two tiles each wrote 64 bytes of every 128-byte line, in 2-byte (248 us) or
+// 8-byte (276) pieces, against 243 now (an 8 s window's QKV GEMM, 49662 x 1568 x
+// 384 on consecutive rows; eight windows' time axis 1694 -> 1655).
+VH_DEVICE uint32_t dpp_quad_xor1(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, false);
+}
+VH_DEVICE uint32_t dpp_quad_xor2(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, false);
+}
+typedef uint32_t kvp_u32x2 __attribute__((ext_vector_type(2)));
+// a: fp16 rows 0 (low half) and 1 of the lane's column, b: rows 2 and 3; the
+// result: row lane % 4, columns 0-3 of the lane's quad.
+VH_DEVICE kvp_u32x2 transpose4_f16(uint32_t a, uint32_t b, int quad) {
+    const uint32_t sel = quad & 1 ? 0x03020706u : 0x05040100u;
+    const uint32_t ca = __builtin_amdgcn_perm(dpp_quad_xor1(a), a, sel);  // row quad & 1, the lane pair's columns
+    const uint32_t cb = __builtin_amdgcn_perm(dpp_quad_xor1(b), b, sel);  // row 2 + (quad & 1)
+    const uint32_t got = dpp_quad_xor2(quad & 2 ? ca : cb);
+    return quad & 2 ? kvp_u32x2{got, cb} : kvp_u32x2{ca, got};
+}
 template <int NJ>
 VH_DEVICE void kv_pieces_epilogue(const GemmDescH2 &d, int row0, int n0, int li, int lh, float2 tv,
-                                  const floatx16 (&acc)[1][NJ], floatx16 rs, floatx4 bpre) {
+                                  const floatx16 (&acc)[1][NJ], floatx16 rs, floatx4 bpre, unsigned char *stage) {
     const bool is_k = n0 < 2 * d.kv_inner;
     const int region = is_k ? d.kv_inner : 2 * d.kv_inner;  // first column of the k (v) region
-    const int B = d.rope_period;
-    // first row (within the wave's 32) of the second frame the rows span: its
-    // table entries are those tv holds in lanes 32-63
-    const int off_b = B - row0 % B;
+    const int quad = li & 3, lane = 32 * lh + li;
     const bool even = (li & 1) == 0;
-    typedef __attribute__((address_space(1))) char gchar;
-    typedef __attribute__((address_space(1))) uint16_t gu16;
+    // column tiles per pass (a head's two, or the wave's one), the bytes of a
+    // row's h or m piece of them and of a staged row, 16-byte slots per row
+    constexpr int TP = NJ >= 2 ? 2 : 1, PIECE = 64 * TP, SPITCH = 2 * PIECE + 16, SLOTS = 2 * PIECE / 16;
+    constexpr int RP = 64 / SLOTS;  // rows per store
+    const float one = opaque_one();
+    char *const rbase = reinterpret_cast<char *>(d.C) + (size_t)row0 * d.ldc * 4u;
     const uint32_t pitch = (uint32_t)d.ldc * 4u;
-    const gchar *const rbase = (const gchar *)(reinterpret_cast<char *>(d.C) + (size_t)row0 * (size_t)pitch);
-    // one straight-line body per (k or v, whole or ragged row tile, frame
-    // boundary inside the wave's rows or not)
-    auto body = [&](auto k_c, auto full_c, auto split_c) {
-        constexpr bool IS_K = decltype(k_c)::value, FULL = decltype(full_c)::value;
-        constexpr bool SPLIT = decltype(split_c)::value;
+    const int p0 = row0 % d.rope_len;  // rope_period 1: the first row's position
+    // rope_period > 1: first row (within the wave's 32) of the second position
+    // the rows span; its table entries are those tv holds in lanes 32-63
+    const int off_b = d.rope_period - row0 % d.rope_period;
+    const int slot = lane % SLOTS, rsub = lane / SLOTS;
+    // one pass at a time: nothing of the next is hoisted into this one (the
+    // registers the K loop needs bound the epilogue's)
 #pragma unroll
-        for (int j = 0; j < NJ; j++) {
-            // one column tile at a time: nothing of the next is hoisted into
-            // this one (the registers the K loop needs bound the epilogue's)
-            __builtin_amdgcn_sched_barrier(0);
-            const int kc = n0 + 32 * j + li - region;
-            const uint32_t off_h = 4u * (uint32_t)region + 256u * (uint32_t)(kc >> 6) + 2u * (uint32_t)(kc & 63) +
-                                   (uint32_t)(4 * lh) * pitch;
-            float c0 = 1.0f, s0 = 0.0f, c1 = 1.0f, s1 = 0.0f;
-            if constexpr (IS_K) {
-                // the lane's pair: its entries from the lanes holding them
-                const int pr = (kc & 63) >> 1;
-                c0 = __shfl(tv.x, pr, 64);
-                s0 = __shfl(tv.y, pr, 64);
-                if (even) s0 = -s0;
-                if constexpr (SPLIT) {
-                    c1 = __shfl(tv.x, 32 + pr, 64);
-                    s1 = __shfl(tv.y, 32 + pr, 64);
-                    if (even) s1 = -s1;
-                }
-            }
-            // rows in pairs (registers r, r + 1: consecutive rows of one
-            // column): one v_cvt_pk_f16_f32 makes both h, one v_fma_mix_f32
-            // per value and one v_cvt_pk_f16_f32 both m (m_pair_f16); the
-            // halves leave by 2-byte stores of each half of the packed dwords
+    for (int jb = 0; jb < NJ; jb += TP) {
+        __builtin_amdgcn_sched_barrier(0);
+        float y[TP][16];
 #pragma unroll
-            for (int r = 0; r < 16; r += 2) {
-                float y[2];
+        for (int jj = 0; jj < TP; jj++)
 #pragma unroll
-                for (int e = 0; e < 2; e++) {
-                    y[e] = fmaf(acc[0][j][r + e], rs[r + e], bpre[j]);
-                    if constexpr (IS_K) {
-                        const float other =
-                            __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(y[e]), 0xB1, 0xF, 0xF, false));
-                        bool nxt = false;
-                        if constexpr (SPLIT) nxt = 8 * ((r + e) >> 2) + 4 * lh + ((r + e) & 3) >= off_b;
-                        y[e] = rope_own(y[e], other, nxt ? c1 : c0, nxt ? s1 : s0);
-                    }
-                }
-                const uint32_t hp = pack_f16x2(y[0], y[1]);
-                const uint32_t mp = m_pair_f16(y[0], y[1], opaque_one(), hp);
+            for (int r = 0; r < 16; r++) y[jj][r] = fmaf(acc[0][jb + jj][r], rs[r], bpre[jb + jj]);
+        if (is_k) {
 #pragma unroll
-                for (int e = 0; e < 2; e++) {
-                    const uint16_t hb = (uint16_t)(hp >> (16 * e)), mb = (uint16_t)(mp >> (16 * e));
-                    const int rr = 8 * ((r + e) >> 2) + ((r + e) & 3);  // the row of register r + e, less 4 lh
-                    if constexpr (FULL) {
-                        // wave-uniform row pointer (SGPRs) + the lane's 32-bit
-                        // offset; the high halves by the d16_hi form of the
-                        // same store, which the compiler would otherwise
-                        // address with a 64-bit VGPR pair per store
-                        const gchar *rp = rbase + (uint32_t)rr * pitch;
-                        asm("" : "+s"(rp));
-                        if (e == 0) {
-                            __builtin_nontemporal_store(hb, (gu16 *)(rp + off_h));
-                            __builtin_nontemporal_store(mb, (gu16 *)(rp + off_h + 128u));
-                        } else {
-                            asm volatile("global_store_short_d16_hi %0, %1, %2 nt\n\t"
-                                         "global_store_short_d16_hi %0, %3, %2 offset:128 nt"
-                                         :
-                                         : "v"(off_h), "v"(hp), "s"(rp), "v"(mp)
-                                         : "memory");
+            for (int jj = 0; jj < TP; jj++) {
+                const int pr = ((n0 + 32 * (jb + jj) + li - region) & 63) >> 1;  // the lane's pair
+                auto turn = [&](int r, float c, float sn) {
+                    const float other =
+                        __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(y[jj][r]), 0xB1, 0xF, 0xF, false));
+                    y[jj][r] = rope_own(y[jj][r], other, c, even ? -sn : sn);
+                };
+                if (d.rope_period == 1) {
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        __builtin_amdgcn_sched_barrier(0);
+                        float2 cs[4];
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            int p = p0 + 8 * q + 4 * lh + e;
+                            if (p >= d.rope_len) p -= d.rope_len;
+                            cs[e] = *reinterpret_cast<const float2 *>(d.rope + 2 * (p * 32 + pr));
                         }
-                    } else if (row0 + rr + 4 * lh < d.M) {
-                        char *rp = reinterpret_cast<char *>(d.C) + (size_t)(row0 + rr) * pitch + off_h;
-                        __builtin_nontemporal_store(hb, reinterpret_cast<uint16_t *>(rp));
-                        __builtin_nontemporal_store(mb, reinterpret_cast<uint16_t *>(rp + 128));
+#pragma unroll
+                        for (int e = 0; e < 4; e++) turn(4 * q + e, cs[e].x, cs[e].y);
+                    }
+                } else {
+                    // the pair's entries from the lanes holding them
+                    const float c0 = __shfl(tv.x, pr, 64), s0 = __shfl(tv.y, pr, 64);
+                    const float c1 = __shfl(tv.x, 32 + pr, 64), s1 = __shfl(tv.y, 32 + pr, 64);
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        const bool nxt = 8 * (r >> 2) + 4 * lh + (r & 3) >= off_b;
+                        turn(r, nxt ? c1 : c0, nxt ? s1 : s0);
                     }
                 }
             }
         }
-    };
-    using T_ = std::true_type;
-    using F_ = std::false_type;
-    if (row0 + 32 <= d.M) {
-        if (!is_k) body(F_(), T_(), F_());
-        else if (off_b >= 32) body(T_(), T_(), F_());
-        else body(T_(), T_(), T_());
-    } else {
-        if (!is_k) body(F_(), F_(), F_());
-        else body(T_(), F_(), T_());
+#pragma unroll
+        for (int jj = 0; jj < TP; jj++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                __builtin_amdgcn_sched_barrier(0);
+                // rows in pairs: one v_cvt_pk_f16_f32 makes both h, one
+                // v_fma_mix_f32 per value and one v_cvt_pk_f16_f32 both m
+                const float *v = &y[jj][4 * q];
+                const uint32_t ha = pack_f16x2(v[0], v[1]), hb = pack_f16x2(v[2], v[3]);
+                const uint32_t ma = m_pair_f16(v[0], v[1], one, ha), mb = m_pair_f16(v[2], v[3], one, hb);
+                unsigned char *const at = stage + (8 * q + 4 * lh + quad) * SPITCH + 64 * jj + 2 * (li & ~3);
+                *reinterpret_cast<kvp_u32x2 *>(at) = transpose4_f16(ha, hb, quad);
+                *reinterpret_cast<kvp_u32x2 *>(at + PIECE) = transpose4_f16(ma, mb, quad);
+            }
+        // the wave's own LDS operations complete in order
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        const int kc = n0 + 32 * jb - region;
+        const uint32_t off = 4u * (uint32_t)region + 256u * (uint32_t)(kc >> 6) + 2u * (uint32_t)(kc & 63) +
+                             (slot < SLOTS / 2 ? 16u * (uint32_t)slot : 128u + 16u * (uint32_t)(slot - SLOTS / 2)) +
+                             (uint32_t)rsub * pitch;
+        typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+        for (int i = 0; i < 32 / RP; i++) {
+            if (i % 2 == 0) __builtin_amdgcn_sched_barrier(0);  // two reads in flight
+            const u32x4 v = *reinterpret_cast<const u32x4 *>(stage + (RP * i + rsub) * SPITCH + 16 * slot);
+            if (row0 + RP * i + rsub < d.M)
+                __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(rbase + (uint32_t)(RP * i) * pitch + off));
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     }
 }
 // Bound on |A|: *ptr when ptr is set (a device float), else value.
@@ -209,7 +234,7 @@ struct H2Tile {
     static constexpr int BM = 32 * WR, BN = 32 * NJ * WC;
     static_assert(BN <= GS_BN && GS_BN % BN == 0, "a tile's columns lie in one 128-row tile of the pieces");
 };
-using H2Tile256 = H2Tile<8, 1, 4, 1, 3, 2>;  // 256 x 128, 72 KB LDS: two workgroups per CU
+using H2Tile256 = H2Tile<8, 1, 4, 1, 3, 4>;  // 256 x 128, 72 KB LDS: two workgroups per CU
 using H2Tile128 = H2Tile<4, 1, 4, 1, 3, 3>;  // 128 x 128, 48 KB: three
 // The small tiles take K 32 at a time (half the barriers: at one wave of work
 // per SIMD between them, they and the LDS latency are the time), which leaves
@@ -342,7 +367,7 @@ __device__ __forceinline__ void gemm_h2_body(const GemmDescH2 &d, float a_bound,
     // loaded now so that their latency is spent in the K loop (two registers)
     float2 tv = make_float2(1.0f, 0.0f);
     if constexpr (KVS && EPI == EPI_STORE) {
-        if (d.kv_pieces && col0 >= d.kv_inner && col0 < 2 * d.kv_inner) {
+        if (d.kv_pieces && d.rope_period > 1 && col0 >= d.kv_inner && col0 < 2 * d.kv_inner) {
             const int f0 = (row0 / d.rope_period) % d.rope_len;
             const int f = lane < 32 ? f0 : (f0 + 1 == d.rope_len ? 0 : f0 + 1);
             tv = *reinterpret_cast<const float2 *>(d.rope + 2 * (f * 32 + (lane & 31)));
@@ -457,8 +482,10 @@ __device__ __forceinline__ void gemm_h2_body(const GemmDescH2 &d, float a_bound,
             // keeps them in registers across the epilogue's variants
             floatx16 rsv;
 #pragma unroll
-            for (int r = 0; r < 16; r++) rsv[r] = NORM ? rs[r] : 1.0f;
-            kv_pieces_epilogue<NJW>(d, row0, col0, li, lh, tv, acc, rsv, floatx4{bpre[0], bpre[1], bpre[2], bpre[3]});
+            for (int r = 0; r < 16; r++) rsv[r] = NORM ? rs[r] : 1.0f;  // x 1 + b: one rounding, as x + b
+            static_assert(RING * STAGE_BYTES / T::WAVES >= 32 * (128 * (NJW >= 2 ? 2 : 1) + 16), "staged rows");
+            kv_pieces_epilogue<NJW>(d, row0, col0, li, lh, tv, acc, rsv, floatx4{bpre[0], bpre[1], bpre[2], bpre[3]},
+                                    ring + wave * (RING * STAGE_BYTES / T::WAVES));
             return;
         }
     }

@@ -389,10 +389,12 @@ static bool gemm_h2_ok(const GemmArgsH2 &g, int epilogue) {
     if (g.row_norm && (g.a_h2 || !(epilogue == EPI_STORE || epilogue == EPI_GELU || epilogue == EPI_GEGLU)))
         return false;
     if (g.amax && epilogue != EPI_RESIDUAL) return false;
-    if (g.kv_inner && (g.kv_inner < 0 || g.kv_inner % 32 || !g.kv_bound || epilogue != EPI_STORE || !g.row_norm))
+    if (g.kv_inner && (g.kv_inner < 0 || g.kv_inner % 32 || !g.kv_bound || epilogue != EPI_STORE ||
+                       !(g.row_norm || g.a_h2)))
         return false;
-    if (g.kv_pieces && (!g.kv_inner || g.kv_inner % 128 || !g.rope || g.rope_period <= 0 || g.rope_len <= 0 ||
-                        3 * g.kv_inner > g.N))
+    // a wave's 32 rows span at most two rotary positions, or 32 consecutive ones
+    if (g.kv_pieces && (!g.kv_inner || g.kv_inner % 128 || !g.rope || g.rope_len <= 0 || 3 * g.kv_inner > g.N ||
+                        (g.rope_period == 1 ? g.rope_len < 32 : g.rope_period < 32)))
         return false;
     return true;
 }
@@ -425,7 +427,7 @@ static void launch_h2(hipStream_t s, const GemmDescH2 &d, const H2Bound &b, cons
         }
     }
     if constexpr (EPI == EPI_STORE) {
-        if (g.kv_inner) {
+        if (g.kv_inner) {  // gemm_h2_ok: h2 rows
             hipLaunchKernelGGL((gemm_h2_kernel<EPI, true, T, false, true>), grid, block, 0, s, d, b);
             return;
         }
@@ -1095,6 +1097,49 @@ bool transformer_block(hipStream_t s, const Dims &d, const LayerWeights &w, floa
     const bool qkv_h2 = use_h2(w.wqkvg_p, D);
     const bool ff1_h2 = use_h2(w.w1_p, D);
     const bool att_h2 = precision == PREC_FP32 && w.bounds && w.att_h2;
+    // the fused projection's k and v columns as the two-piece attention takes
+    // them; false: plain fp32
+    auto kv_out = [&](GemmArgsH2 &gq) {
+        // L in (64, 128]: one query group per sequence and head, so nothing
+        // done once here is repeated by the attention, and the plain epilogue
+        // is the cheaper one (862 x 90, D = 256, QKV + attention: 439 us plain
+        // or prescaled, 473 as pieces)
+        if (lay.L > 64 && lay.L <= 128) return false;
+        // k and v written times the attention's piece scales, so its staging
+        // splits them without a multiply (the same bits: VOCALARC_KV_PRESCALE=0
+        // keeps them unscaled, to check that)
+        const char *kv_env = getenv("VOCALARC_KV_PRESCALE");
+        if (!att_h2 || inner % 32 || (kv_env && kv_env[0] == '0')) return false;
+        gq.kv_bound = w.bounds + 1;
+        gq.kv_inner = inner;
+        // On long axes k (rotated) and v leave the QKV GEMM as the attention's
+        // fp16 pieces, which it copies into LDS without computing
+        // (attention_h2_kvp_kernel): the rotation and the split happen once
+        // per element instead of once per query group.  Row orders whose
+        // position the epilogue finds from the row number: [..][position]
+        // [sequence] with at least 32 sequences beside each other (the time
+        // axis of [chunk][frame][band], the band axis of [band][frame]), and
+        // sequences of consecutive rows.  QKV + attention of 62 x 801
+        // consecutive rows, D = 384: 562 us without, 542 with; 90 x 862, D =
+        // 256: 693 without, 645 with.  VOCALARC_KV_PIECES=0 keeps k and v fp32
+        // (the same bits).
+        const char *kvp_env = getenv("VOCALARC_KV_PIECES");
+        const bool rows_interleaved = lay.seq_stride == 1 && lay.pos_stride == lay.group && lay.group >= 32 &&
+                                      (lay.S <= lay.group || lay.group_stride == lay.group * lay.L) &&
+                                      lay.S % lay.group == 0;
+        const bool rows_consecutive = lay.pos_stride == 1 && lay.group == 1 && lay.group_stride == lay.L;
+        const bool off32 = tokens * nq * 4 <= (int64_t)UINT32_MAX;  // its staging offsets, as attention() checks
+        const bool kv_pieces = lay.L > 64 && inner % 128 == 0 && tokens == (int64_t)lay.S * lay.L &&
+                               (rows_interleaved || rows_consecutive) && off32 &&
+                               !(kvp_env && kvp_env[0] == '0');
+        if (kv_pieces) {
+            gq.kv_pieces = true;
+            gq.rope = rt;
+            gq.rope_period = rows_interleaved ? lay.group : 1;
+            gq.rope_len = lay.L;
+        }
+        return true;
+    };
     if (xb && xb->dev && xb->scratch && qkv_h2 && ff1_h2 && w.wqkvg_pg && use_h2(w.wout_p, inner) &&
         use_h2(w.w2_p, d.ff_dim)) {
         // The attention's pre-norm inside the QKV GEMM (row_norm, the gain in
@@ -1109,30 +1154,7 @@ bool transformer_block(hipStream_t s, const Dims &d, const LayerWeights &w, floa
         xb->valid = false;  // until the FFN down-projection has raised the slot
         GemmArgsH2 gq{x, D, w.wqkvg_pg, w.bqkvg, qkvg, nq, tokens, nq, D};
         gq.row_norm = true;
-        // k and v written times the attention's piece scales, so its staging
-        // splits them without a multiply (the same bits: VOCALARC_KV_PRESCALE=0
-        // keeps them unscaled, to check that)
-        const char *kv_env = getenv("VOCALARC_KV_PRESCALE");
-        const bool kv_pre = att_h2 && inner % 32 == 0 && !(kv_env && kv_env[0] == '0');
-        if (kv_pre) {
-            gq.kv_bound = w.bounds + 1;
-            gq.kv_inner = inner;
-        }
-        // On the time axis of the [chunk][frame][band] token order, k (rotated)
-        // and v leave the QKV GEMM as the attention's fp16 pieces, which it
-        // copies into LDS without computing (attention_h2_kvp_kernel): the
-        // rotation and the split happen once per element instead of once per
-        // query group.  VOCALARC_KV_PIECES=0 keeps them fp32 (the same bits).
-        const char *kvp_env = getenv("VOCALARC_KV_PIECES");
-        const bool kv_pieces = kv_pre && lay.L > 64 && inner % 128 == 0 && lay.seq_stride == 1 &&
-                               lay.pos_stride == lay.group && lay.group_stride == lay.group * lay.L &&
-                               !(kvp_env && kvp_env[0] == '0');
-        if (kv_pieces) {
-            gq.kv_pieces = true;
-            gq.rope = rt;
-            gq.rope_period = lay.group;
-            gq.rope_len = lay.L;
-        }
+        const bool kv_pre = kv_out(gq), kv_pieces = gq.kv_pieces;
         // On the band axis (sequences of L <= 64 consecutive rows) the
         // projection and the attention run as one kernel (band_attention.hpp):
         // q, k, v and the gate logits stay on chip.  VOCALARC_BAND_FUSED=0
@@ -1172,14 +1194,23 @@ bool transformer_block(hipStream_t s, const Dims &d, const LayerWeights &w, floa
     if (!(qkv_h2 ? rmsnorm_h2(s, x, D, w.gamma, normed, D, tokens, D, w.bounds, t)
                  : rmsnorm(s, x, D, w.gamma, normed, D, tokens, D, t)))
         return false;
-    if (!lin(normed, D, w.wqkvg, w.wqkvg_p, 0, w.bqkvg, qkvg, nq, nq, D, EPI_STORE, qkv_h2, "gemm_qkv")) return false;
+    bool kv_pre = false, kv_pieces = false;
+    if (qkv_h2) {
+        GemmArgsH2 gq{normed, D, w.wqkvg_p, w.bqkvg, qkvg, nq, tokens, nq, D};
+        gq.a_h2 = true;
+        kv_pre = kv_out(gq);
+        kv_pieces = gq.kv_pieces;
+        if (!gemm_h2(s, gq, OperandBound{w.bounds, 0.0f}, EPI_STORE, t, "gemm_qkv")) return false;
+    } else if (!lin(normed, D, w.wqkvg, nullptr, 0, w.bqkvg, qkvg, nq, nq, D, EPI_STORE, false, "gemm_qkv")) {
+        return false;
+    }
     // rotary + attention + gates (products as fp16 two-piece splits on the
     // default fp32 path)
     // the two-piece attention writes its output as the out projection's
     // pieces when that GEMM runs on them (same bound: the value bound)
     const bool attn_rows = att_h2 && use_h2(w.wout_p, inner);
     if (!attention(s, qkvg, nq, attn, inner, rt, lay, d.heads, gate, t, false, false, precision == PREC_FP32,
-                   att_h2 ? w.bounds + 1 : nullptr, attn_rows))
+                   att_h2 ? w.bounds + 1 : nullptr, attn_rows, kv_pre, false, kv_pieces))
         return false;
     // out projection added to the residual stream
     if (!lin(attn, inner, w.wout, w.wout_p, 1, nullptr, x, D, D, inner, EPI_RESIDUAL, attn_rows, "gemm_out"))

@@ -142,14 +142,14 @@ struct GemmArgsH2 {
     bool row_norm = false;
     float *zero_slot = nullptr;  // a device float the kernel sets to 0
     float *amax = nullptr;       // EPI_RESIDUAL: raised to max |C| written
-    // kv_inner > 0 (a multiple of 32; EPI_STORE with row_norm): C is a fused
+    // kv_inner > 0 (a multiple of 32; EPI_STORE with row_norm or a_h2): C is a fused
     // q|k|v|gates projection whose k and v columns are written times 2^ek and
     // 2^ev of the attention bound *kv_bound (GemmDescH2::kv_inner)
     const float *kv_bound = nullptr;
     int kv_inner = 0;
     // with kv_inner (a multiple of 128): k (rotated by the interleaved table
-    // rope of rope_len positions, row r at frame (r / rope_period) % rope_len)
-    // and v written as fp16 pieces for attention(kv_pieces) (GemmDescH2)
+    // rope of rope_len positions, row r at position (r / rope_period) %
+    // rope_len; rope_period 1 with rope_len >= 32, or >= 32) and v written as fp16 pieces for attention(kv_pieces) (GemmDescH2)
     bool kv_pieces = false;
     const float *rope = nullptr;
     int rope_period = 0, rope_len = 0;

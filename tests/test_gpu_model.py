@@ -112,6 +112,26 @@ def test_band_attention_fused(cfg2_models, rng, monkeypatch, S, L):
     assert snr_db(outs[1], outs[0]) >= 120.0
 
 
+@pytest.mark.parametrize("axis,S,L", [(0, 3, 129), (1, 5, 160), (0, 2, 801), (0, 31, 191)])
+def test_kv_pieces_consecutive_rows_bit_identical(cfg2_models, rng, monkeypatch, axis, S, L):
+    """A block on sequences of consecutive rows (vh_transformer's order): the QKV GEMM rotates k by one position
+    per row, sequences ending inside a wave's 32 rows, and a ragged last row tile; the same bits as the attention's own
+    rotation and split (VOCALARC_KV_PIECES=0)."""
+    om, dm = cfg2_models
+    x = rng.standard_normal((S, L, om.d.dim), dtype=np.float32)
+    outs = []
+    for env in (None, "0"):
+        if env is None:
+            monkeypatch.delenv("VOCALARC_KV_PIECES", raising=False)
+        else:
+            monkeypatch.setenv("VOCALARC_KV_PIECES", env)
+        dx = to_dev(x)
+        dm.transformer(1, axis, dx, S, L)
+        outs.append(from_dev(dx))
+    monkeypatch.delenv("VOCALARC_KV_PIECES", raising=False)
+    assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+
+
 @pytest.mark.parametrize("windows", [1, 3])
 def test_kv_pieces_bit_identical(cfg2_models, monkeypatch, windows):
     """On the pipeline's time axis (L > 64, [chunk][frame][band] rows) the
