@@ -683,7 +683,12 @@ bool stage_stft(vh_model *m, const float *audio, int64_t audio_len, const int64_
     a.C = d.channels; a.T = T; a.F = d.freq_bins(); a.n_fft = d.n_fft; a.log2n = log2i(d.n_fft); a.hop = d.hop;
     a.window = m->window.f(); a.tw = static_cast<const double2_t *>(m->twiddle.ptr); a.source = source; a.out = lay;
     Scope sc(&m->ctx->timer, m->ctx->stream, "stft");
-    hipLaunchKernelGGL(stft_kernel, dim3(T, chunks * d.channels), dim3(256), fft_lds_bytes(d.n_fft), m->ctx->stream, a);
+    if (d.n_fft == RF_N)
+        hipLaunchKernelGGL(stft2048_kernel, dim3((T + RF_FRAMES - 1) / RF_FRAMES, chunks * d.channels),
+                           dim3(64 * RF_FRAMES), 0, m->ctx->stream, a);
+    else
+        hipLaunchKernelGGL(stft_kernel, dim3(T, chunks * d.channels), dim3(256), fft_lds_bytes(d.n_fft), m->ctx->stream,
+                           a);
     return sync_debug(m->ctx->stream, "stft_kernel");
 }
 
@@ -823,7 +828,11 @@ bool stage_istft(vh_model *m, const float *source, const float *mask, const Spec
     a.log2n = log2i(d.n_fft); a.window = m->window.f(); a.tw = static_cast<const double2_t *>(m->twiddle.ptr);
     a.frames = m->frames.f();
     Scope sc(&m->ctx->timer, s, "istft");
-    hipLaunchKernelGGL(istft_frames_kernel, dim3(T, sigs), dim3(256), fft_lds_bytes(d.n_fft), s, a);
+    if (d.n_fft == RF_N)
+        hipLaunchKernelGGL(istft2048_frames_kernel, dim3((T + RF_FRAMES - 1) / RF_FRAMES, sigs), dim3(64 * RF_FRAMES), 0,
+                           s, a);
+    else
+        hipLaunchKernelGGL(istft_frames_kernel, dim3(T, sigs), dim3(256), fft_lds_bytes(d.n_fft), s, a);
     if (!sync_debug(s, "istft_frames_kernel")) return false;
     OlaArgs o;
     o.frames = m->frames.f(); o.window = m->window.f(); o.T = T; o.n_fft = d.n_fft; o.hop = d.hop; o.length = length;

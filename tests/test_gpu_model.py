@@ -208,6 +208,30 @@ def test_stft_istft(ctx, cfg2_models, ref_models, which, layout):
     assert T == src.shape[2]
 
 
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("length", [1200, 2049, 3969, 4410])
+def test_stft_istft_edges(cfg2_models, rng, length, layout):
+    """Signals of a few frames (3, 5, 9 or 11: the kernels take four at a time), reflected at both ends, digital
+    silence in the first half of one channel, and a mask that makes bins 0 and 1024 complex (only their real parts
+    reach the signal)."""
+    om, dm = cfg2_models
+    d = om.d
+    x = rng.standard_normal((d.channels, length)).astype(np.float32)
+    x[0, :length // 2] = 0.0
+    src = O.stft(d, x)
+    dsrc = empty_dev(_to_layout(src, layout).shape)
+    dm.stft(to_dev(x), length, dsrc, layout)
+    got = _from_layout(from_dev(dsrc), layout)
+    assert_close(src, got, rtol=1e-6, atol=4e-6, min_snr=120, what="stft")
+    silent = [t for t in range(src.shape[2]) if not np.any(src[:, 0, t])]
+    assert np.all(got[:, 0, silent] == 0.0)  # an exactly silent frame stays exactly zero
+    mask = rng.standard_normal(src.shape).astype(np.float32)
+    ref = O.istft(d, src, mask, length)
+    dout = empty_dev((d.channels, length))
+    dm.istft(to_dev(_to_layout(src, layout)), to_dev(_to_layout(mask, layout)), length, dout, layout)
+    assert_close(ref, from_dev(dout), rtol=1e-5, atol=4e-6, min_snr=120, what="istft")
+
+
 def test_istft_perfect_reconstruction(ctx, cfg2_models):
     """A unit mask reproduces the input (closed form: Hann OLA normalised by
     the summed squared window)."""
