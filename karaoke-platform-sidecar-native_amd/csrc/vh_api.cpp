@@ -9,6 +9,7 @@
 #include <mutex>
 #include <vector>
 
+#include "band_split.hpp"
 #include "dsp.hpp"
 #include "elementwise.hpp"
 #include "runtime.hpp"
@@ -61,6 +62,11 @@ struct vh_model {
     DeviceBuffer weights_s, bounds;
     std::vector<void *> mask_w1_s, mask_w2_s;
     std::vector<void *> band_w_h, mask_w1_h, mask_w2_h;
+    // the band split's pieces (built at load; band_split.hpp): per band one
+    // descriptor, and the bands by the rows' width (band_split_kernel's
+    // KMAX); no descriptors: the gather and the fp32 MFMA GEMM run instead
+    DeviceBuffer band_pieces, band_descs;
+    std::vector<int> band_class[3];
     // DSP constants
     DeviceBuffer window, twiddle;
     // pipeline scratch (grown on demand)
@@ -653,6 +659,79 @@ bool prepare_split(vh_model *m) {
     return check(hipStreamSynchronize(s), "hipStreamSynchronize(split weights)");
 }
 
+// The band split's descriptors: weight pieces and gains padded to K chunks of
+// 16, the exponent of each band's normalised rows.
+constexpr int BAND_CLASS_K[3] = {192, 528, 640};
+bool prepare_band_split(vh_model *m) {
+    const Dims &d = m->d;
+    hipStream_t s = m->ctx->stream;
+    const int B = d.bands, D = d.dim;
+    auto kpad = [&](int b) { return (d.in_dim(b) + GS_BK - 1) / GS_BK * GS_BK; };
+    auto round = [](size_t n) { return (n + 255) & ~(size_t)255; };
+    size_t total = round(2 * (size_t)B * sizeof(float)), widest = 0;
+    for (int b = 0; b < B; b++) {
+        total += round(h2_bytes(D, kpad(b))) + round(kpad(b) * sizeof(float));
+        widest = std::max(widest, (size_t)D * kpad(b) * sizeof(float));
+        if (kpad(b) > BAND_CLASS_K[2]) return true;
+    }
+    DeviceBuffer padded;  // a weight matrix widened to its K chunks
+    if (!m->band_pieces.ensure(total, "hipMalloc(band pieces)") || !padded.ensure(widest, "hipMalloc(padded band weight)") ||
+        !check(hipMemsetAsync(m->band_pieces.ptr, 0, total, s), "hipMemset(band pieces)"))
+        return false;
+    char *cur = static_cast<char *>(m->band_pieces.ptr);
+    float *bounds = reinterpret_cast<float *>(cur);
+    cur += round(2 * (size_t)B * sizeof(float));
+    std::vector<BandSplitDesc> descs(B);
+    for (int b = 0; b < B; b++) {
+        const int K = d.in_dim(b), P = kpad(b);
+        BandSplitDesc &e = descs[b];
+        e.W = cur;
+        const float *W = m->band_w[b];
+        if (P != K) {
+            if (!check(hipMemsetAsync(padded.ptr, 0, (size_t)D * P * sizeof(float), s), "hipMemset(padded band weight)") ||
+                !check(hipMemcpy2DAsync(padded.ptr, P * sizeof(float), W, K * sizeof(float), K * sizeof(float), D,
+                                        hipMemcpyDeviceToDevice, s), "hipMemcpy2D(band weight)"))
+                return false;
+            W = padded.f();
+        }
+        if (!split_weights_h2(s, W, D, P, P, cur)) return false;
+        cur += round(h2_bytes(D, P));
+        e.gamma = reinterpret_cast<float *>(cur);
+        if (!check(hipMemcpyAsync(cur, m->band_gamma[b], K * sizeof(float), hipMemcpyDeviceToDevice, s),
+                   "hipMemcpy(band gain)"))
+            return false;
+        cur += round(P * sizeof(float));
+        e.bias = m->band_b[b];
+        e.first_freq = m->first_freq[b];
+        e.width = d.band_widths[b];
+        e.kpad = P;
+        if (!operand_bounds(s, m->band_gamma[b], K, nullptr, 0, nullptr, false, bounds + 2 * b)) return false;
+    }
+    std::vector<float> host(2 * (size_t)B);
+    if (!check(hipMemcpyAsync(host.data(), bounds, host.size() * sizeof(float), hipMemcpyDeviceToHost, s),
+               "hipMemcpy(band bounds)") ||
+        !check(hipStreamSynchronize(s), "hipStreamSynchronize(band bounds)"))
+        return false;
+    std::vector<int> list;
+    for (int b = 0; b < B; b++) {
+        // beyond the scale range: the band split stays on fp32 MFMA
+        if (!(host[2 * b] >= 0.0f && host[2 * b] <= 1.0e30f)) return true;
+        descs[b].ea = h2_exponent(host[2 * b]);
+    }
+    for (int c = 0; c < 3; c++) {
+        for (int b = 0; b < B; b++)
+            if (descs[b].kpad <= BAND_CLASS_K[c] && (c == 0 || descs[b].kpad > BAND_CLASS_K[c - 1]))
+                m->band_class[c].push_back(b);
+        list.insert(list.end(), m->band_class[c].begin(), m->band_class[c].end());
+    }
+    const size_t db = B * sizeof(BandSplitDesc);
+    return m->band_descs.ensure(db + B * sizeof(int), "hipMalloc(band descriptors)") &&
+           check(hipMemcpyAsync(m->band_descs.ptr, descs.data(), db, hipMemcpyHostToDevice, s), "hipMemcpy(band descriptors)") &&
+           check(hipMemcpyAsync(static_cast<char *>(m->band_descs.ptr) + db, list.data(), B * sizeof(int),
+                                hipMemcpyHostToDevice, s), "hipMemcpy(band list)") &&
+           check(hipStreamSynchronize(s), "hipStreamSynchronize(band descriptors)");
+}
+
 // Batched token-wise linears of one pipeline stage in the model's precision
 // (fp32 activations; the bf16 variant rounds them as they are staged).
 bool stage_gemms(vh_model *m, const std::vector<GemmArgs> &gs, const std::vector<void *> &wh, int epi,
@@ -699,6 +778,30 @@ bool stage_band_split(vh_model *m, const float *source, const SpecLayout &lay, i
     const Dims &d = m->d;
     hipStream_t s = m->ctx->stream;
     const int M = chunks * T, B = d.bands, D = d.dim;
+    if (m->precision == PREC_FP32 && m->band_descs.ptr) {
+        BandSplitArgs a;
+        a.source = source; a.lay = lay;
+        a.bands = static_cast<const BandSplitDesc *>(m->band_descs.ptr);
+        const int *list = reinterpret_cast<const int *>(a.bands + B);
+        a.out = out;
+        a.band_stride = frame_major ? D : (int64_t)M * D;
+        a.ldo = frame_major ? (int64_t)B * D : D;
+        a.M = M; a.T = T; a.C = d.channels; a.D = D;
+        Scope sc(&m->ctx->timer, s, "gemm_band_split");
+        for (int c = 0; c < 3; c++) {
+            a.list = list;
+            a.count = (int)m->band_class[c].size();
+            list += a.count;
+            if (!a.count) continue;
+            const int rt = c == 0 ? 64 : 32;
+            const dim3 grid((unsigned)((M + rt - 1) / rt) * (unsigned)a.count), block(BS_THREADS);
+            if (c == 0) hipLaunchKernelGGL((band_split_kernel<64, BAND_CLASS_K[0], 3>), grid, block, 0, s, a);
+            else if (c == 1) hipLaunchKernelGGL((band_split_kernel<32, BAND_CLASS_K[1], 2>), grid, block, 0, s, a);
+            else hipLaunchKernelGGL((band_split_kernel<32, BAND_CLASS_K[2], 2>), grid, block, 0, s, a);
+            if (!sync_debug(s, "band_split_kernel")) return false;
+        }
+        return true;
+    }
     if (!m->bandin.ensure((size_t)M * m->band_in_total * sizeof(float), "hipMalloc(band input)") ||
         !m->tables.ensure(sizeof(BandTable) + sizeof(MaskTable), "hipMalloc(tables)"))
         return false;
@@ -902,7 +1005,7 @@ extern "C" vh_model *vh_model_load(vh_context *ctx, const vh_dims *dims, const v
         delete m;
         return nullptr;
     }
-    if (!upload_pack(m, pack, bytes) || !prepare_split(m)) {
+    if (!upload_pack(m, pack, bytes) || !prepare_split(m) || !prepare_band_split(m)) {
         delete m;
         return nullptr;
     }

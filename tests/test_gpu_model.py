@@ -268,6 +268,29 @@ def test_band_split_and_mask(ctx, cfg2_models, ref_models, which, rng, layout):
                  what="mask estimator")
 
 
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("T", [1, 31, 33, 65, 130])
+@pytest.mark.parametrize("which", ["config", "reference"])
+def test_band_split_and_mask_row_tiles(cfg2_models, ref_models, which, rng, T, layout):
+    """Frames around the kernels' 32 and 64 row tiles, of very different level (the rows are normalised before
+    they are split into fp16 pieces, so quiet frames keep their precision) and one of zeros; the mask's GLU and
+    scatter on ragged row tiles, bands of 8 to 516 inputs (16-wide value and gate groups)."""
+    om, dm = cfg2_models if which == "config" else ref_models
+    d = om.d
+    src = rng.standard_normal((d.freq_bins, d.channels, T, 2)).astype(np.float32)
+    src *= (10.0 ** rng.uniform(-5, 4, T)).astype(np.float32)[None, None, :, None]
+    src[:, :, T // 2] = 0.0
+    ref = om.band_split(src)
+    dout = empty_dev(ref.shape)
+    dm.band_split(to_dev(_to_layout(src, layout)), T, dout, layout)
+    assert_close(ref, from_dev(dout), rtol=1e-4, atol=2e-5, min_snr=110, what="band split")
+    feats = rng.standard_normal((T, d.bands, d.dim), dtype=np.float32)
+    mref = om.mask_estimate(feats)
+    dmask = empty_dev(_to_layout(mref, layout).shape)
+    dm.mask_estimate(to_dev(feats), T, dmask, layout)
+    assert_close(mref, _from_layout(from_dev(dmask), layout), rtol=1e-4, atol=1e-5, min_snr=110, what="mask")
+
+
 def test_forward_config_shape(cfg2_models):
     om, dm = cfg2_models
     x = audio.sine_mix(0.5, 11)
