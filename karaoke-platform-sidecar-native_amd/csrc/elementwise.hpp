@@ -331,7 +331,7 @@ static __global__ __launch_bounds__(256) void band_gather_norm_kernel(const floa
 struct MaskTable {
     int first_freq[256];
     int dim[256];            // 4w
-    int64_t proj_offset[256];
+    int64_t proj_offset[256];  // float offset of the band's projection per row (times the rows: its first)
 };
 
 static __global__ __launch_bounds__(256) void mask_glu_scatter_kernel(const float *__restrict__ proj,
@@ -344,11 +344,21 @@ static __global__ __launch_bounds__(256) void mask_glu_scatter_kernel(const floa
     if (e >= (int64_t)M * dim) return;
     const int m = (int)(e / dim), i = (int)(e % dim);
     const int chunk = m / T, t = m % T;
-    const float *p = proj + tab->proj_offset[b] + (size_t)m * 2 * dim;
+    const float *p = proj + tab->proj_offset[b] * M + (size_t)m * 2 * dim;
     const float val = p[i] * (1.0f / (1.0f + __expf(-p[dim + i])));
     const int f = tab->first_freq[b] + i / (2 * C);
     const int c = (i / 2) % C, comp = i & 1;
     mask[2 * spec_at(lay, chunk, f, c, t) + comp] = val;
+}
+
+// [2 dim][K] (values, then gates) -> rows in (16 value, 16 gate) groups, zero past dim
+static __global__ __launch_bounds__(256) void glu16_rows_kernel(const float *__restrict__ src, float *__restrict__ dst,
+                                                         int dim, int K, int64_t n) {
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e >= n) return;
+    const int r = (int)(e / K), k = (int)(e % K);
+    const int i = r / 32 * 16 + r % 16;
+    dst[e] = i < dim ? src[(size_t)(r % 32 < 16 ? i : dim + i) * K + k] : 0.0f;
 }
 
 }  // namespace vh

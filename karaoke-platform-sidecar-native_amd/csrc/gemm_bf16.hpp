@@ -131,7 +131,7 @@ VH_DEVICE void gemm_bf16_epilogue(const GemmDescBF16 &d, const floatx16 (&acc)[F
                 auto value = [&](int r) {
                     const float v = pre(i, j, r, bc);
                     if constexpr (EPI == EPI_GELU) return gelu_dev(v);
-                    else if constexpr (EPI == EPI_TANH) return tanhf(v);
+                    else if constexpr (EPI == EPI_TANH) return tanh_dev(v);
                     else return v;
                 };
                 if (rows_full) {
@@ -374,7 +374,7 @@ VH_DEVICE void gemm_bf16_epilogue_staged(const GemmDescBF16 &d, const floatx16 (
                     for (int e = 0; e < 4; e++) {
                         o[e] = v[e] + b[e];
                         if constexpr (EPI == EPI_GELU) o[e] = gelu_dev(o[e]);
-                        else if constexpr (EPI == EPI_TANH) o[e] = tanhf(o[e]);
+                        else if constexpr (EPI == EPI_TANH) o[e] = tanh_dev(o[e]);
                     }
                     *reinterpret_cast<bf16x4 *>(&stage[(32 * i + li) * PITCH + c]) = to_bf16x4(o);
                 }

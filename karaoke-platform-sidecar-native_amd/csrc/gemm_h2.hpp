@@ -79,7 +79,50 @@ struct GemmDescH2 {
     int kv_pieces;
     const float *rope;
     int rope_period, rope_len;
+    // EPI_MASK_GLU: the band's first frequency and its inputs
+    int mask_f0, mask_dim;
 };
+// EPI_MASK_GLU: where the mask goes.
+struct H2MaskOut {
+    float *mask;
+    SpecLayout lay;
+    int T, C;
+};
+
+// The mask estimator's GLU and bin scatter on a wave's 32 x 32 NJ tile of its
+// second layer, whose columns come in (16 value, 16 gate) groups.  Of two
+// accumulator rows r, r + 1 v_permlane16_swap leaves the values of r in lanes
+// 0-15 and of r + 1 in lanes 16-31 of one register, their gates in the other:
+// every lane then holds one output.  The projection (twice the mask's bytes)
+// is no longer written, read back and scattered by a pass of its own (36 us of
+// 474 on an 8 s window).
+template <int NJ>
+VH_DEVICE void mask_glu_epilogue(const GemmDescH2 &d, const H2MaskOut &o, int row0, int col0, int li, int lh,
+                                 const floatx16 (&acc)[1][NJ], const float *bpre) {
+    const int ch0 = row0 / o.T, t0 = row0 - ch0 * o.T;
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+        const int i = (col0 + 32 * j) / 2 + (li & 15);
+        const int pair = i >> 1, f = pair / o.C, c = pair - f * o.C;
+        const int64_t at = spec_at(o.lay, 0, d.mask_f0 + f, c, 0);
+#pragma unroll
+        for (int r = 0; r < 16; r += 2) {
+            typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+            const u32x2 vg = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[0][j][r] + bpre[j]),
+                                                              __float_as_uint(acc[0][j][r + 1] + bpre[j]), false, false);
+            const float v = __uint_as_float(vg[0]) * sigmoid_dev(__uint_as_float(vg[1]));
+            const int off = 8 * (r >> 2) + 4 * lh + (r & 3) + (li >> 4);
+            int t = t0 + off, ch = ch0;
+            while (t >= o.T) {
+                t -= o.T;
+                ch++;
+            }
+            if (i < d.mask_dim && row0 + off < d.M)
+                o.mask[2 * (at + ch * o.lay.chunk_s + t * o.lay.t_s) + (i & 1)] = v;
+        }
+    }
+}
+
 
 // The fused projection's k or v column tile (32 x 32 NJ per wave, n0 inside
 // [kv_inner, 3 kv_inner)) written as fp16 pieces instead of fp32: the head's
@@ -260,7 +303,8 @@ constexpr int H2_WBLOCK = 2 * GS_BN * GS_BK;  // fp16 per (row tile, K chunk) bl
 // the fused projection's instantiations, and with kv_pieces written as their
 // fp16 pieces (k rotated).
 template <int EPI, bool A_H2, class T, bool NORM = false, bool KVS = false>
-__device__ __forceinline__ void gemm_h2_body(const GemmDescH2 &d, float a_bound, int tile) {
+__device__ __forceinline__ void gemm_h2_body(const GemmDescH2 &d, float a_bound, int tile,
+                                             const H2MaskOut *mo = nullptr) {
     static_assert(!(NORM && A_H2), "the row norm needs the fp32 rows");
     static_assert(EPI != EPI_GEGLU || T::NJ % 2 == 0, "a wave holds the value and the gate columns");
     constexpr int NJW = T::NJ, RING = T::RING, KS = T::KS;
@@ -489,6 +533,10 @@ __device__ __forceinline__ void gemm_h2_body(const GemmDescH2 &d, float a_bound,
             return;
         }
     }
+    if constexpr (EPI == EPI_MASK_GLU) {
+        mask_glu_epilogue<NJW>(d, *mo, row0, col0, li, lh, acc, bpre);
+        return;
+    }
     GemmDescBF16 e{};
     e.bias = d.bias; e.C = d.C; e.M = d.M; e.N = d.N; e.K = d.K; e.ldc = d.ldc;
     float mx = 0.0f;
@@ -521,11 +569,12 @@ __global__ __launch_bounds__(T::THREADS, T::OCC) void gemm_h2_kernel(GemmDescH2 
 struct GemmBatchH2 {
     GemmDescH2 d[GS_MAX_BATCH];
     H2Bound b;
+    H2MaskOut mo;  // EPI_MASK_GLU
 };
 
 template <int EPI, class T>
 __global__ __launch_bounds__(T::THREADS, T::OCC) void gemm_h2_batched_kernel(GemmBatchH2 b) {
-    gemm_h2_body<EPI, false, T>(b.d[blockIdx.z], b.b.ptr ? *b.b.ptr : b.b.value, (int)blockIdx.x);
+    gemm_h2_body<EPI, false, T>(b.d[blockIdx.z], b.b.ptr ? *b.b.ptr : b.b.value, (int)blockIdx.x, &b.mo);
 }
 
 // max |W| over W [N][ldw] (first K columns) into out[0]; one workgroup of

@@ -564,7 +564,7 @@ extern "C" int native_gpu_resident_mask(native_gpu *gpu, int frames, const float
         s2.push_back({hid, Hm, w2s, b2, gpu->proj.f() + off, 2 * dim, M, 2 * dim, Hm});
         tab.first_freq[b] = bands[b].first_frequency;
         tab.dim[b] = dim;
-        tab.proj_offset[b] = off;
+        tab.proj_offset[b] = off / M;
         off += (int64_t)M * 2 * dim;
         maxdim = std::max(maxdim, dim);
     }

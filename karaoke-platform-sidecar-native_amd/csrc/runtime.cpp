@@ -408,6 +408,7 @@ static GemmDescH2 to_desc_h2(const GemmArgsH2 &g) {
     d.kv_bound = g.kv_bound; d.kv_inner = g.kv_inner;
     d.kv_pieces = g.kv_pieces ? 1 : 0;
     d.rope = g.rope; d.rope_period = g.rope_period; d.rope_len = g.rope_len;
+    d.mask_f0 = d.mask_dim = 0;
     return d;
 }
 
@@ -620,6 +621,38 @@ bool gemm_h2_batched(hipStream_t s, const std::vector<GemmArgsH2> &gs, const Ope
         if (!sync_debug(s, "gemm_h2_batched_kernel")) return false;
     }
     return true;
+}
+
+bool gemm_h2_mask(hipStream_t s, const std::vector<MaskBandH2> &bands, int64_t M, const OperandBound &bound, float *mask,
+                  const SpecLayout &lay, int T, int C, KernelTimer *t, const char *name) {
+    Scope sc(t, s, name);
+    for (size_t first = 0; first < bands.size(); first += GS_MAX_BATCH) {
+        const size_t count = std::min(bands.size() - first, (size_t)GS_MAX_BATCH);
+        GemmBatchH2 b;
+        memset(&b, 0, sizeof(b));
+        b.b = H2Bound{bound.dev, bound.value};
+        b.mo = H2MaskOut{mask, lay, T, C};
+        for (size_t i = 0; i < count; i++) {
+            const MaskBandH2 &m = bands[first + i];
+            const GemmArgsH2 g{m.A, m.lda, m.W, m.bias, mask, glu16_width(m.dim), M, glu16_width(m.dim), m.K};
+            if (!gemm_h2_ok(g, EPI_MASK_GLU) || m.dim <= 0 || T <= 0 || C <= 0) {
+                set_error("gemm_h2_mask: unsupported shape M=%lld dim=%d K=%d lda=%d", (long long)M, m.dim, m.K, m.lda);
+                return false;
+            }
+            b.d[i] = to_desc_h2(g);
+            b.d[i].mask_f0 = m.first_freq;
+            b.d[i].mask_dim = m.dim;
+        }
+        launch_h2_batched<EPI_MASK_GLU>(s, b, (unsigned)count);
+        if (!sync_debug(s, "gemm_h2_batched_kernel (mask)")) return false;
+    }
+    return true;
+}
+
+bool glu16_rows(hipStream_t s, const float *src, float *dst, int dim, int K) {
+    const int64_t n = (int64_t)glu16_width(dim) * K;
+    hipLaunchKernelGGL(glu16_rows_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, s, src, dst, dim, K, n);
+    return sync_debug(s, "glu16_rows_kernel");
 }
 
 bool split_weights_h2(hipStream_t s, const float *W, int N, int K, int ldw, void *pieces) {

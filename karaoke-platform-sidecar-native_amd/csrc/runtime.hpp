@@ -14,6 +14,8 @@
 
 #include "../../include/vocalarc_hip.h"
 
+struct SpecLayout;  // common.hpp
+
 namespace vh {
 
 // ----------------------------------------------------------------- errors
@@ -76,6 +78,7 @@ enum Epilogue : int {
     EPI_TANH = 2,      // C = tanh(acc + bias)
     EPI_RESIDUAL = 3,  // C += acc + bias
     EPI_GEGLU = 4,     // columns come in (32 value, 32 gate) pairs: C[:, n/2] = v * gelu(g)
+    EPI_MASK_GLU = 5,  // gemm_h2_mask only: (16 value, 16 gate) pairs, v * sigmoid(g) scattered into the mask
 };
 
 struct GemmArgs {
@@ -163,6 +166,23 @@ bool gemm_h2(hipStream_t s, const GemmArgsH2 &g, const OperandBound &bound, int 
 // A ragged batch of fp16 two-piece GEMMs with one A bound (one launch per 64 problems).
 bool gemm_h2_batched(hipStream_t s, const std::vector<GemmArgsH2> &gs, const OperandBound &bound, int epilogue,
                      KernelTimer *t = nullptr, const char *name = "gemm_h2");
+// The mask estimator's second layer with its GLU and the reference's bin
+// scatter: per band A [M][K], W and bias with their rows in (16 value, 16 gate)
+// groups (glu16_rows, N = glu16_width(dim)), value i of row m written to bin
+// (frequency first_freq + i / 2C, channel (i / 2) % C, component i % 2) of
+// chunk m / T, frame m % T of mask in layout lay.
+struct MaskBandH2 {
+    const float *A; int lda;
+    const void *W;
+    const float *bias;
+    int K, dim, first_freq;
+};
+bool gemm_h2_mask(hipStream_t s, const std::vector<MaskBandH2> &bands, int64_t M, const OperandBound &bound, float *mask,
+                  const SpecLayout &lay, int T, int C, KernelTimer *t = nullptr, const char *name = "gemm_mask2");
+inline int glu16_width(int dim) { return (dim + 15) / 16 * 32; }
+// src [2 dim][K] (values, then gates) -> dst [glu16_width(dim)][K], rows in
+// (16 value, 16 gate) groups, zero past dim.
+bool glu16_rows(hipStream_t s, const float *src, float *dst, int dim, int K);
 // The band-axis attention fused with its pre-norm projection
 // (band_attention.hpp): for S sequences of L <= 64 consecutive rows of the
 // residual stream x, the q, k, v and gate columns of the gain-folded fused

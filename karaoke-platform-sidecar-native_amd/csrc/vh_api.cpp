@@ -60,7 +60,9 @@ struct vh_model {
     // (layer_bounds), then the mask estimator's feature bound, then absmax
     // scratch
     DeviceBuffer weights_s, bounds;
-    std::vector<void *> mask_w1_s, mask_w2_s;
+    std::vector<void *> mask_w1_s, mask_w2_s;  // w2: rows in (16 value, 16 gate) groups (gemm_h2_mask)
+    std::vector<float *> mask_b2_s;            // and its bias
+    DeviceBuffer mask_table;                   // MaskTable (mask_glu_scatter_kernel)
     std::vector<void *> band_w_h, mask_w1_h, mask_w2_h;
     // the band split's pieces (built at load; band_split.hpp): per band one
     // descriptor, and the bands by the rows' width (band_split_kernel's
@@ -544,6 +546,18 @@ bool upload_pack(vh_model *m, const void *pack, size_t bytes) {
         m->band_in_total += d.in_dim(k);
         m->proj_total += 2 * d.in_dim(k);
     }
+    MaskTable tab;
+    memset(&tab, 0, sizeof(tab));
+    int64_t off = 0;
+    for (int k = 0; k < d.bands; k++) {
+        tab.first_freq[k] = m->first_freq[k];
+        tab.dim[k] = d.in_dim(k);
+        tab.proj_offset[k] = off;
+        off += 2 * d.in_dim(k);
+    }
+    if (!m->mask_table.ensure(sizeof(tab), "hipMalloc(mask table)") ||
+        !check(hipMemcpyAsync(m->mask_table.ptr, &tab, sizeof(tab), hipMemcpyHostToDevice, s), "hipMemcpy(mask table)"))
+        return false;
     return check(hipStreamSynchronize(s), "hipStreamSynchronize(model upload)");
 }
 
@@ -605,7 +619,9 @@ bool prepare_split(vh_model *m) {
     const size_t per_layer = 2 * bytes(d.qkvg_dim(), D) + bytes(D, d.inner()) + bytes(d.ff1_out(), D) +
                              bytes(D, d.ff_dim) + gate_bytes;
     size_t total = per_layer * m->layers.size();
-    for (int b = 0; b < d.bands; b++) total += bytes(Hm, D) + bytes(2 * d.in_dim(b), Hm);
+    auto glu_bias = [&](int b) { return ((size_t)glu16_width(d.in_dim(b)) * sizeof(float) + 255) & ~(size_t)255; };
+    for (int b = 0; b < d.bands; b++) total += bytes(Hm, D) + bytes(glu16_width(d.in_dim(b)), Hm) + glu_bias(b);
+    m->mask_b2_s.assign(d.bands, nullptr);
     m->mask_w1_s.assign(d.bands, nullptr);
     m->mask_w2_s.assign(d.bands, nullptr);
     if (!m->bounds.ensure((4 * m->layers.size() + 64 + ABSMAX_PARTIALS) * sizeof(float), "hipMalloc(operand bounds)"))
@@ -654,8 +670,15 @@ bool prepare_split(vh_model *m) {
         }
     }
     for (int b = 0; b < d.bands && mask_ok; b++)  // no pieces: the mask estimator stays on fp32 MFMA
-        if (!split(m->mask_w1[b], Hm, D, &m->mask_w1_s[b]) || !split(m->mask_w2[b], 2 * d.in_dim(b), Hm, &m->mask_w2_s[b]))
+    {
+        const int dim = d.in_dim(b), N = glu16_width(dim);
+        if (!fold_tmp.ensure((size_t)N * Hm * sizeof(float), "hipMalloc(mask weight)")) return false;
+        m->mask_b2_s[b] = reinterpret_cast<float *>(cur);
+        cur += glu_bias(b);
+        if (!split(m->mask_w1[b], Hm, D, &m->mask_w1_s[b]) || !glu16_rows(s, m->mask_b2[b], m->mask_b2_s[b], dim, 1) ||
+            !glu16_rows(s, m->mask_w2[b], fold_tmp.f(), dim, Hm) || !split(fold_tmp.f(), N, Hm, &m->mask_w2_s[b]))
             return false;
+    }
     return check(hipStreamSynchronize(s), "hipStreamSynchronize(split weights)");
 }
 
@@ -803,7 +826,7 @@ bool stage_band_split(vh_model *m, const float *source, const SpecLayout &lay, i
         return true;
     }
     if (!m->bandin.ensure((size_t)M * m->band_in_total * sizeof(float), "hipMalloc(band input)") ||
-        !m->tables.ensure(sizeof(BandTable) + sizeof(MaskTable), "hipMalloc(tables)"))
+        !m->tables.ensure(sizeof(BandTable), "hipMalloc(band table)"))
         return false;
     BandTable tab;
     memset(&tab, 0, sizeof(tab));
@@ -845,18 +868,16 @@ bool stage_mask(vh_model *m, const void *normed, bool normed_bf16, int chunks, i
         return false;
     }
     const size_t hid_elem = h ? 2 : 4, feat_elem = normed_bf16 ? 2 : 4;  // the bf16 hidden layer feeds layer 2 as is
-    if (!m->mhidden.ensure((size_t)B * M * Hm * hid_elem, "hipMalloc(mask hidden)") ||
-        !m->proj.ensure((size_t)M * m->proj_total * sizeof(float), "hipMalloc(mask projection)") ||
-        !m->tables.ensure(sizeof(BandTable) + sizeof(MaskTable), "hipMalloc(tables)"))
-        return false;
+    if (!m->mhidden.ensure((size_t)B * M * Hm * hid_elem, "hipMalloc(mask hidden)")) return false;
     std::vector<GemmArgs> g1, g2;
     std::vector<GemmArgsBF16> h1, h2;
-    std::vector<GemmArgsH2> s1, s2;
-    // fp32 path: both layers on the fp16 two-piece GEMM when every band's pieces exist
+    std::vector<GemmArgsH2> s1;
+    std::vector<MaskBandH2> s2;
+    // fp32 path: both layers on the fp16 two-piece GEMM when every band's pieces
+    // exist, the second with the GLU and the scatter in its epilogue
     bool sp = m->precision == PREC_FP32 && !normed_bf16;
     for (int b = 0; b < B && sp; b++) sp = m->mask_w1_s.size() == (size_t)B && m->mask_w1_s[b] && m->mask_w2_s[b];
-    MaskTable tab;
-    memset(&tab, 0, sizeof(tab));
+    if (!sp && !m->proj.ensure((size_t)M * m->proj_total * sizeof(float), "hipMalloc(mask projection)")) return false;
     int64_t off = 0;
     for (int b = 0; b < B; b++) {
         char *hid = static_cast<char *>(m->mhidden.ptr) + (size_t)b * M * Hm * hid_elem;
@@ -874,17 +895,14 @@ bool stage_mask(vh_model *m, const void *normed, bool normed_bf16, int chunks, i
         } else if (sp) {
             s1.push_back({reinterpret_cast<const float *>(feat), B * D, m->mask_w1_s[b], m->mask_b1[b],
                           reinterpret_cast<float *>(hid), Hm, M, Hm, D});
-            s2.push_back({reinterpret_cast<const float *>(hid), Hm, m->mask_w2_s[b], m->mask_b2[b], proj, out, M, out,
-                          Hm});
+            s2.push_back({reinterpret_cast<const float *>(hid), Hm, m->mask_w2_s[b], m->mask_b2_s[b], Hm, d.in_dim(b),
+                          m->first_freq[b]});
         } else {
             g1.push_back({reinterpret_cast<const float *>(feat), B * D, m->mask_w1[b], D, m->mask_b1[b],
                           reinterpret_cast<float *>(hid), Hm, M, Hm, D});
             g2.push_back({reinterpret_cast<const float *>(hid), Hm, m->mask_w2[b], Hm, m->mask_b2[b], proj, out, M, out,
                           Hm});
         }
-        tab.first_freq[b] = m->first_freq[b];
-        tab.dim[b] = d.in_dim(b);
-        tab.proj_offset[b] = off;
         off += (int64_t)M * out;
     }
     KernelTimer *t = &m->ctx->timer;
@@ -900,23 +918,19 @@ bool stage_mask(vh_model *m, const void *normed, bool normed_bf16, int chunks, i
             if (!absmax(s, static_cast<const float *>(normed), (int64_t)M * B * D, absmax_scratch(m), fb)) return false;
             b1.dev = fb;
         }
-        if (!gemm_h2_batched(s, s1, b1, EPI_TANH, t, "gemm_mask1") ||
-            !gemm_h2_batched(s, s2, OperandBound{nullptr, 1.0f}, EPI_STORE, t, "gemm_mask2"))
-            return false;
+        return gemm_h2_batched(s, s1, b1, EPI_TANH, t, "gemm_mask1") &&
+               gemm_h2_mask(s, s2, M, OperandBound{nullptr, 1.0f}, mask, lay, T, d.channels, t);
     } else if (!gemm_batched(s, g1, EPI_TANH, t, "gemm_mask1") || !gemm_batched(s, g2, EPI_STORE, t, "gemm_mask2")) {
         return false;
     }
-    MaskTable *dtab = reinterpret_cast<MaskTable *>(static_cast<char *>(m->tables.ptr) + sizeof(BandTable));
-    if (!check(hipMemcpyAsync(dtab, &tab, sizeof(tab), hipMemcpyHostToDevice, s), "hipMemcpy(mask table)")) return false;
     int maxdim = 0;
     for (int b = 0; b < B; b++) maxdim = std::max(maxdim, d.in_dim(b));
     {
         Scope sc(&m->ctx->timer, s, "mask_glu");
         hipLaunchKernelGGL(mask_glu_scatter_kernel, dim3((unsigned)(((int64_t)M * maxdim + 255) / 256), B), dim3(256), 0, s,
-                           m->proj.f(), dtab, mask, lay, M, T, d.channels);
-        if (!sync_debug(s, "mask_glu_scatter_kernel")) return false;
+                           m->proj.f(), static_cast<const MaskTable *>(m->mask_table.ptr), mask, lay, M, T, d.channels);
+        return sync_debug(s, "mask_glu_scatter_kernel");
     }
-    return check(hipStreamSynchronize(s), "hipStreamSynchronize(mask table)");
 }
 
 // source, mask (layout lay) -> out[chunks*C][pitch] (first `length` samples of each)
