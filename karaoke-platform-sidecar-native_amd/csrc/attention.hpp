@@ -57,7 +57,8 @@ struct AttnArgs {
     const float *guard;
     int guard_h2;
     // k and v arrive as the fused projection's fp16 pieces
-    // (GemmDescH2::kv_pieces; attention_h2_kvp_kernel)
+    // (GemmDescH2::kv_pieces; attention_h2_kvp_kernel); bf16 qkv: k arrives
+    // rotated (GemmDescBF16::rope; attention_bf16_kvp_kernel)
     int kv_pieces;
 };
 
@@ -100,6 +101,23 @@ VH_DEVICE floatx4 rope4_table(floatx4 v, const float *tab, int pos, int d0) {
 }
 VH_DEVICE floatx4 rope4(floatx4 v, const float *tab, int pos, int d0) {
     return tab == nullptr ? v : rope4_table(v, tab, pos, d0);
+}
+
+VH_DEVICE floatx4 lo4(bf16x8 v) { return floatx4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]}; }
+VH_DEVICE floatx4 hi4(bf16x8 v) { return floatx4{(float)v[4], (float)v[5], (float)v[6], (float)v[7]}; }
+
+// Rotate the four interleaved pairs of 8 dims starting at d0 (fp32), scale,
+// round to bf16.
+VH_DEVICE bf16x8 rope8_bf16(bf16x8 v, const float *tab, int pos, int d0, float scale) {
+    floatx4 a = rope4(lo4(v), tab, pos, d0) * scale;
+    floatx4 b = rope4(hi4(v), tab, pos, d0 + 4) * scale;
+    bf16x8 r;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        r[e] = (bf16)a[e];
+        r[4 + e] = (bf16)b[e];
+    }
+    return r;
 }
 
 // Workgroup: WAVES wavefronts x 32 queries of one (sequence, head).  Each

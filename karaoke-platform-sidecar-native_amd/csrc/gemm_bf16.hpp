@@ -19,6 +19,7 @@
 
 #include <type_traits>
 
+#include "attention.hpp"
 #include "common.hpp"
 
 namespace vh {
@@ -30,6 +31,13 @@ struct GemmDescBF16 {
     void *C;            // fp32 or bf16 [M][ldc]
     int M, N, K;
     int lda, ldb, ldc;
+    // rope (staged bf16 store only; null for none): columns [rope_inner, 2
+    // rope_inner) are heads of 64 dims and leave rotated -- each finished,
+    // rounded value pair turned in fp32 and rounded again, as the attention
+    // would do when it stages k -- row r at position (r / rope_period) %
+    // rope_len of the interleaved table (rope_period 1, or >= 32)
+    const float *rope;
+    int rope_inner, rope_period, rope_len;
 };
 
 constexpr int GB_MAX_BATCH = 64;
@@ -386,6 +394,23 @@ VH_DEVICE void gemm_bf16_epilogue_staged(const GemmDescBF16 &d, const floatx16 (
     const int oc0 = EPI == EPI_GEGLU ? col0 / 2 : col0;
     const int ncols = EPI == EPI_GEGLU ? d.N / 2 : d.N;
     bf16 *C = static_cast<bf16 *>(d.C);
+    // k's columns: the lane's eight dims of row row0 + rr rotated
+    const bool turn = EPI == EPI_STORE && d.rope && oc0 >= d.rope_inner && oc0 < 2 * d.rope_inner;
+    const int per = turn && d.rope_period > 1 ? d.rope_period : 1;
+    const int p0 = turn ? row0 / per % d.rope_len : 0, n0 = turn ? row0 % per : 0;
+    auto rotated = [&](bf16x8 v, int rr) {
+        int p = p0, n = n0 + rr;
+        if (per == 1) {
+            p += rr;
+        } else {
+            while (n >= per) {
+                n -= per;
+                p++;
+            }
+        }
+        while (p >= d.rope_len) p -= d.rope_len;
+        return rope8_bf16(v, d.rope, p, 8 * (lane % LPR), 1.0f);
+    };
     if (row0 + 64 <= d.M && oc0 + OC <= ncols) {
         // whole block inside C: the store of rows RPI t .. from a row pointer
         // the wave shares (SGPRs, kept opaque as in gemm_bf16_epilogue) plus
@@ -396,7 +421,10 @@ VH_DEVICE void gemm_bf16_epilogue_staged(const GemmDescBF16 &d, const floatx16 (
         const gchar *rbase = (const gchar *)(reinterpret_cast<char *>(C) + (size_t)row0 * (size_t)pitch);
 #pragma unroll
         for (int t = 0; t < 64 / RPI; t++) {
-            const bf16x8 v = *reinterpret_cast<const bf16x8 *>(&stage[(RPI * t + lane / LPR) * PITCH + 8 * (lane % LPR)]);
+            bf16x8 v = *reinterpret_cast<const bf16x8 *>(&stage[(RPI * t + lane / LPR) * PITCH + 8 * (lane % LPR)]);
+            if constexpr (EPI == EPI_STORE) {
+                if (turn) v = rotated(v, RPI * t + lane / LPR);
+            }
             const gchar *rp = rbase + (uint32_t)(RPI * t) * pitch;
             asm("" : "+s"(rp));
             *(__attribute__((address_space(1))) bf16x8 *)(rp + off) = v;
@@ -406,7 +434,10 @@ VH_DEVICE void gemm_bf16_epilogue_staged(const GemmDescBF16 &d, const floatx16 (
 #pragma unroll
     for (int t = 0; t < 64 / RPI; t++) {
         const int rr = RPI * t + lane / LPR, c8 = 8 * (lane % LPR);
-        const bf16x8 v = *reinterpret_cast<const bf16x8 *>(&stage[rr * PITCH + c8]);
+        bf16x8 v = *reinterpret_cast<const bf16x8 *>(&stage[rr * PITCH + c8]);
+        if constexpr (EPI == EPI_STORE) {
+            if (turn) v = rotated(v, rr);
+        }
         const int row = row0 + rr, col = oc0 + c8;
         if (row < d.M) {
             bf16 *dst = C + (size_t)row * d.ldc + col;
@@ -453,14 +484,17 @@ VH_DEVICE void wait_vmcnt() {
     asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
 }
 
+// Blocks of 64 WM x 128: 2 WM waves.  WM = 4 (256 x 128, 72 KB, two workgroups
+// per CU) where a launch fills the chip several times over, WM = 2 (128 x 128,
+// 48 KB, three) where its tiles divide more evenly (the launcher's rule).
 constexpr int GBD_BM = 256, GBD_BN = 128, GBD_BK = 32, GBD_STAGES = 3, GBD_THREADS = 512;
 
-template <int EPI, typename TC>
+template <int EPI, typename TC, int WM>
 __device__ __forceinline__ void gemm_bf16_dma_body(const GemmDescBF16 &d, int tile) {
     // bf16 outputs leave through LDS in row order (gemm_bf16_epilogue_staged):
     // their MFMAs take the B tile first
     constexpr bool ROWS = std::is_same<TC, bf16>::value;
-    constexpr int BM = GBD_BM, BN = GBD_BN, BK = GBD_BK, STAGES = GBD_STAGES, W = GBD_THREADS / 64;
+    constexpr int BM = 64 * WM, BN = GBD_BN, BK = GBD_BK, STAGES = GBD_STAGES, W = 2 * WM;
     constexpr int A_BYTES = BM * BK * 2, STAGE_BYTES = A_BYTES + BN * BK * 2;
     constexpr int NA = BM / 16 / W, NB = BN / 16 / W;  // load instructions per wave per chunk
     static_assert(NA * 16 * W == BM && NB * 16 * W == BN, "loads must tile the chunk");
@@ -469,7 +503,7 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmDescBF16 &d, int ti
     const int tiles_n = (d.N + BN - 1) / BN;
     const int tiles_m = (d.M + BM - 1) / BM;
     if (tile >= tiles_m * tiles_n) return;
-    const int gsz = (size_t)d.N * d.K * sizeof(bf16) <= (3u << 20) ? 1 : 8;
+    const int gsz = (size_t)d.N * d.K * sizeof(bf16) <= (3u << 20) ? 1 : 2048 / BM;
     const int group = tile / (gsz * tiles_n);
     const int in_group = tile % (gsz * tiles_n);
     const int group_rows = min(gsz, tiles_m - group * gsz);
@@ -478,7 +512,7 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmDescBF16 &d, int ti
 
     const int tid = (int)threadIdx.x;
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
-    const int wm = wave >> 1, wn = wave & 1;  // 4 x 2 waves of 64 x 64
+    const int wm = wave >> 1, wn = wave & 1;  // WM x 2 waves of 64 x 64
     const int li = lane & 31, lh = lane >> 5;
     const uint32_t ring_base = (uint32_t)(uintptr_t)ring;
     auto swz = [](int r) { return (r >> 2) & 3; };
@@ -565,7 +599,7 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmDescBF16 &d, int ti
     if constexpr (ROWS) {
         // the ring is free: every wave finished its reads before the last
         // barrier and no load is in flight; wave w stages in its own ninth
-        static_assert(GBD_THREADS / 64 * 64 * (64 + 8) * 2 <= STAGES * STAGE_BYTES, "staging fits the ring");
+        static_assert(W * 64 * (64 + 8) * 2 <= STAGES * STAGE_BYTES, "staging fits the ring");
         gemm_bf16_epilogue_staged<EPI>(d, acc, reinterpret_cast<bf16 *>(ring) + wave * 64 * (64 + 8), m0 + wm * 64,
                                        n0 + wn * 64, lane, bq);
     } else {
@@ -573,14 +607,14 @@ __device__ __forceinline__ void gemm_bf16_dma_body(const GemmDescBF16 &d, int ti
     }
 }
 
-template <int EPI, typename TC>
-__global__ __launch_bounds__(GBD_THREADS, 2) void gemm_bf16_dma_kernel(GemmDescBF16 d) {
-    gemm_bf16_dma_body<EPI, TC>(d, xcd_swizzle((int)blockIdx.x, (int)gridDim.x));
+template <int EPI, typename TC, int WM>
+__global__ __launch_bounds__(128 * WM, WM == 4 ? 2 : 3) void gemm_bf16_dma_kernel(GemmDescBF16 d) {
+    gemm_bf16_dma_body<EPI, TC, WM>(d, xcd_swizzle((int)blockIdx.x, (int)gridDim.x));
 }
 
 template <int EPI, typename TC>
 __global__ __launch_bounds__(GBD_THREADS, 2) void gemm_bf16_dma_batched_kernel(GemmBatchBF16 b) {
-    gemm_bf16_dma_body<EPI, TC>(b.d[blockIdx.z], (int)blockIdx.x);
+    gemm_bf16_dma_body<EPI, TC, 4>(b.d[blockIdx.z], (int)blockIdx.x);
 }
 
 // fp32 [rows][cols] -> bf16 [rows][ld] (weights at upload; padding untouched)

@@ -196,6 +196,13 @@ bool gemm_batched(hipStream_t s, const std::vector<GemmArgs> &gs, int epilogue, 
     return true;
 }
 
+// CUs of the device (256 on an MI355X).
+static int device_cus() {
+    static int cus = 0;
+    if (cus == 0 && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, 0) != hipSuccess) cus = 256;
+    return cus;
+}
+
 // ------------------------------------------------------------ bf16 GEMM
 static bool gemm_bf16_ok(const GemmArgsBF16 &g, int epilogue) {
     if (g.M <= 0 || g.N <= 0 || g.K <= 0 || g.M > INT32_MAX / 2) return false;
@@ -205,6 +212,10 @@ static bool gemm_bf16_ok(const GemmArgsBF16 &g, int epilogue) {
     if (g.ldc < out_cols(g.N, epilogue) || g.ldc > (1 << 21) || (epilogue == EPI_GEGLU && g.N % 64)) return false;
     if (g.c_bf16 && epilogue == EPI_RESIDUAL) return false;
     if (((uintptr_t)g.A | (uintptr_t)g.B) & 15) return false;
+    if (g.rope && (epilogue != EPI_STORE || !g.c_bf16 || !g.a_bf16 || g.staged || g.K % GBD_BK || g.lda > (1 << 21) ||
+                   g.ldb > (1 << 21) || g.rope_inner <= 0 || g.rope_inner % 64 || 2 * g.rope_inner > g.N ||
+                   g.rope_len <= 0 || (g.rope_period != 1 && g.rope_period < 32)))
+        return false;
     return true;
 }
 
@@ -213,6 +224,7 @@ static GemmDescBF16 to_desc_bf16(const GemmArgsBF16 &g) {
     d.A = g.A; d.B = static_cast<const bf16 *>(g.B); d.bias = g.bias; d.C = g.C;
     d.M = (int)g.M; d.N = g.N; d.K = g.K;
     d.lda = g.lda; d.ldb = g.ldb; d.ldc = g.ldc;
+    d.rope = g.rope; d.rope_inner = g.rope_inner; d.rope_period = g.rope_period; d.rope_len = g.rope_len;
     return d;
 }
 
@@ -242,9 +254,22 @@ static void launch_bf16_typed(hipStream_t s, const GemmDescBF16 *single, const G
                               unsigned n, bool dma) {
     if constexpr (std::is_same<TA, bf16>::value) {
         if (dma) {
-            if (single)
-                hipLaunchKernelGGL((gemm_bf16_dma_kernel<EPI, TC>), dim3(tiles), dim3(GBD_THREADS), 0, s, *single);
-            else
+            if (single) {
+                // 128-row blocks where their finer division of the launch over
+                // the CUs outweighs their 8% higher cost per element (as
+                // h2_tile_pick; N = 384: K = 512 and 1536 at 49662 rows
+                // 104 us each on 256 rows, @@ on 128)
+                auto per_cu = [&](int bm) {
+                    const int64_t t = (int64_t)((single->M + bm - 1) / bm) * ((single->N + GBD_BN - 1) / GBD_BN);
+                    return (double)((t + device_cus() - 1) / device_cus());
+                };
+                if (std::max(per_cu(128) * 1.08, 1.47) < per_cu(256) * 2.0)
+                    hipLaunchKernelGGL((gemm_bf16_dma_kernel<EPI, TC, 2>),
+                                       dim3((unsigned)((single->M + 127) / 128) * (unsigned)((single->N + GBD_BN - 1) / GBD_BN)),
+                                       dim3(256), 0, s, *single);
+                else
+                    hipLaunchKernelGGL((gemm_bf16_dma_kernel<EPI, TC, 4>), dim3(tiles), dim3(GBD_THREADS), 0, s, *single);
+            } else
                 hipLaunchKernelGGL((gemm_bf16_dma_batched_kernel<EPI, TC>), dim3(tiles, 1, n), dim3(GBD_THREADS), 0,
                                    s, *batch);
             return;
@@ -435,13 +460,6 @@ static void launch_h2(hipStream_t s, const GemmDescH2 &d, const H2Bound &b, cons
     }
     if (g.a_h2) hipLaunchKernelGGL((gemm_h2_kernel<EPI, true, T>), grid, block, 0, s, d, b);
     else hipLaunchKernelGGL((gemm_h2_kernel<EPI, false, T>), grid, block, 0, s, d, b);
-}
-
-// CUs of the device (256 on an MI355X).
-static int device_cus() {
-    static int cus = 0;
-    if (cus == 0 && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, 0) != hipSuccess) cus = 256;
-    return cus;
 }
 
 // The block tile of a two-piece GEMM launch: the one of the least modelled
@@ -900,6 +918,13 @@ static void launch_attention(hipStream_t s, const AttnArgs &a, unsigned grid, bo
             return;
         }
     }
+    if constexpr (WAVES == 4) {
+        if (qkv_bf16 && a.kv_pieces) {  // attention() checked the offsets
+            if (out_bf16) hipLaunchKernelGGL((attention_bf16_kvp_kernel<bf16>), dim3(grid), block, 0, s, a);
+            else hipLaunchKernelGGL((attention_bf16_kvp_kernel<float>), dim3(grid), block, 0, s, a);
+            return;
+        }
+    }
     if (qkv_bf16) {
         if (out_bf16) hipLaunchKernelGGL((attention_bf16_kernel<WAVES, bf16>), dim3(grid), block, 0, s, a);
         else hipLaunchKernelGGL((attention_bf16_kernel<WAVES, float>), dim3(grid), block, 0, s, a);
@@ -930,8 +955,13 @@ bool attention(hipStream_t s, const void *qkv, int ld, void *out, int ld_out, co
                                  (int64_t)(std::min(lay.S, lay.group) - 1) * lay.seq_stride +
                                  (int64_t)(lay.L - 1) * lay.pos_stride;
         const bool off32 = lay.group_stride >= 0 && lay.seq_stride >= 0 && lay.pos_stride >= 0 &&
-                           (last_row + 1) * ld * 4 <= (int64_t)UINT32_MAX;
-        if (!kv_scaled || lay.L <= 64 || !rope || heads * ATT_DH % 128 || device_choice || out_bf16 || !off32) {
+                           (last_row + 1) * ld * (qkv_bf16 ? 2 : 4) <= (int64_t)UINT32_MAX;
+        if (qkv_bf16) {
+            if (lay.L <= 64 || !rope || kv_scaled || device_choice || !off32) {
+                set_error("attention: rotated bf16 k needs L > 64, the rotary table and 32-bit staging offsets");
+                return false;
+            }
+        } else if (!kv_scaled || lay.L <= 64 || !rope || heads * ATT_DH % 128 || device_choice || out_bf16 || !off32) {
             set_error("attention: k/v pieces need the prescaled two-piece kernel, L > 64, fp32 out, the rotary "
                       "table and 32-bit staging offsets");
             return false;
@@ -1090,6 +1120,15 @@ bool transformer_block(hipStream_t s, const Dims &d, const LayerWeights &w, floa
     float *normed = scr.normed.f(), *qkvg = scr.qkvg.f(), *attn = scr.attn.f(), *hid = scr.hidden.f();
     const int gate = d.gated ? d.qkv_dim() : -1;
     const int ff1_epi = d.ffn_glu ? EPI_GEGLU : EPI_GELU;
+    // Row orders whose rotary position a GEMM epilogue finds from the row
+    // number: [..][position][sequence] with at least 32 sequences beside each
+    // other (the time axis of [chunk][frame][band], the band axis of
+    // [band][frame]), and sequences of consecutive rows.  0: neither.
+    const bool rows_interleaved = lay.seq_stride == 1 && lay.pos_stride == lay.group && lay.group >= 32 &&
+                                  (lay.S <= lay.group || lay.group_stride == lay.group * lay.L) &&
+                                  lay.S % lay.group == 0;
+    const bool rows_consecutive = lay.pos_stride == 1 && lay.group == 1 && lay.group_stride == lay.L;
+    const int rope_period = tokens != (int64_t)lay.S * lay.L ? 0 : rows_interleaved ? lay.group : rows_consecutive ? 1 : 0;
     if (precision == PREC_BF16) {
         // bf16 variant: the normalised activations, the fused projection, the
         // attention output and the FFN hidden layer are stored as bf16 -- the
@@ -1106,8 +1145,24 @@ bool transformer_block(hipStream_t s, const Dims &d, const LayerWeights &w, floa
             return gemm_bf16(s, g, epi, t, name);
         };
         if (!rmsnorm_bf16(s, x, D, w.gamma, normed, D, tokens, D, t)) return false;
-        if (!lin(normed, D, w.wqkvg_h, w.bqkvg, qkvg, nq, nq, D, EPI_STORE, true, "gemm_qkv")) return false;
-        if (!attention(s, qkvg, nq, attn, inner, rt, lay, d.heads, gate, t, true, true)) return false;
+        // more than one query group per sequence: k leaves the projection
+        // rotated and the attention stages it without computing (the same bits;
+        // VOCALARC_KV_PIECES=0 keeps k unrotated)
+        const char *kvp_env = getenv("VOCALARC_KV_PIECES");
+        const bool k_rotated = lay.L > 128 && rope_period && D % 32 == 0 && tokens * nq * 2 <= (int64_t)UINT32_MAX &&
+                               !(kvp_env && kvp_env[0] == '0');
+        GemmArgsBF16 gq{normed, D, w.wqkvg_h, bf16_pitch(D), w.bqkvg, qkvg, nq, tokens, nq, D};
+        gq.a_bf16 = gq.c_bf16 = true;
+        if (k_rotated) {
+            gq.rope = rt;
+            gq.rope_inner = inner;
+            gq.rope_period = rope_period;
+            gq.rope_len = lay.L;
+        }
+        if (!gemm_bf16(s, gq, EPI_STORE, t, "gemm_qkv")) return false;
+        if (!attention(s, qkvg, nq, attn, inner, rt, lay, d.heads, gate, t, true, true, false, nullptr, false, false,
+                       false, k_rotated))
+            return false;
         if (!lin(attn, inner, w.wout_h, nullptr, x, D, D, inner, EPI_RESIDUAL, false, "gemm_out")) return false;
         if (!rmsnorm_bf16(s, x, D, w.ff_gamma, normed, D, tokens, D, t)) return false;
         if (!lin(normed, D, w.w1_h, w.b1, hid, d.ff_dim, d.ff1_out(), D, ff1_epi, true, "gemm_ff1")) return false;
@@ -1148,27 +1203,18 @@ bool transformer_block(hipStream_t s, const Dims &d, const LayerWeights &w, floa
         // On long axes k (rotated) and v leave the QKV GEMM as the attention's
         // fp16 pieces, which it copies into LDS without computing
         // (attention_h2_kvp_kernel): the rotation and the split happen once
-        // per element instead of once per query group.  Row orders whose
-        // position the epilogue finds from the row number: [..][position]
-        // [sequence] with at least 32 sequences beside each other (the time
-        // axis of [chunk][frame][band], the band axis of [band][frame]), and
-        // sequences of consecutive rows.  QKV + attention of 62 x 801
+        // per element instead of once per query group.  QKV + attention of 62 x 801
         // consecutive rows, D = 384: 562 us without, 542 with; 90 x 862, D =
         // 256: 693 without, 645 with.  VOCALARC_KV_PIECES=0 keeps k and v fp32
         // (the same bits).
         const char *kvp_env = getenv("VOCALARC_KV_PIECES");
-        const bool rows_interleaved = lay.seq_stride == 1 && lay.pos_stride == lay.group && lay.group >= 32 &&
-                                      (lay.S <= lay.group || lay.group_stride == lay.group * lay.L) &&
-                                      lay.S % lay.group == 0;
-        const bool rows_consecutive = lay.pos_stride == 1 && lay.group == 1 && lay.group_stride == lay.L;
         const bool off32 = tokens * nq * 4 <= (int64_t)UINT32_MAX;  // its staging offsets, as attention() checks
-        const bool kv_pieces = lay.L > 64 && inner % 128 == 0 && tokens == (int64_t)lay.S * lay.L &&
-                               (rows_interleaved || rows_consecutive) && off32 &&
-                               !(kvp_env && kvp_env[0] == '0');
+        const bool kv_pieces =
+            lay.L > 64 && inner % 128 == 0 && rope_period && off32 && !(kvp_env && kvp_env[0] == '0');
         if (kv_pieces) {
             gq.kv_pieces = true;
             gq.rope = rt;
-            gq.rope_period = rows_interleaved ? lay.group : 1;
+            gq.rope_period = rope_period;
             gq.rope_len = lay.L;
         }
         return true;

@@ -103,6 +103,11 @@ struct GemmArgsBF16 {
     int64_t M; int N, K;
     bool a_bf16 = false, c_bf16 = false;
     bool staged = false;     // bf16 A with K % 32 == 0: force the register-staged kernel over the DMA ring
+    // columns [rope_inner, 2 rope_inner) (a multiple of 64) rotated by the
+    // interleaved table, row r at position (r / rope_period) % rope_len,
+    // rope_period 1 or >= 32 (EPI_STORE, bf16 A and C, K % 32 == 0); null: none
+    const float *rope = nullptr;
+    int rope_inner = 0, rope_period = 0, rope_len = 0;
 };
 bool gemm_bf16(hipStream_t s, const GemmArgsBF16 &g, int epilogue, KernelTimer *t = nullptr,
                const char *name = "gemm_bf16");
@@ -269,7 +274,8 @@ struct AttnLayout {
 // launched, each returning at once unless the bound's range selects it
 // (AttnArgs::guard), so the call never synchronises.
 // kv_pieces (with kv_scaled, L > 64): k and v arrive as the fp16 pieces a
-// gemm_h2 with kv_pieces writes (k rotated; rope must be the table it used).
+// gemm_h2 with kv_pieces writes (k rotated; rope must be the table it used);
+// with qkv_bf16: k arrives rotated, as a gemm_bf16 with rope writes it.
 bool attention(hipStream_t s, const void *qkv, int ld, void *out, int ld_out, const float *rope, const AttnLayout &lay,
                int heads, int gate_col, KernelTimer *t = nullptr, bool out_bf16 = false, bool qkv_bf16 = false,
                bool split = false, const float *bound = nullptr, bool out_h2 = false, bool kv_scaled = false,

@@ -376,23 +376,23 @@ def main() -> int:
             fm = native.SPEC_FRAME_MAJOR
             src = torch.empty(d.channels, Tf, d.freq_bins, 2, device=dev)
             _emit("stft", _event_time(lambda: model.stft(x, length, src, fm), reps),
-                  gbytes=(x.numel() + src.numel()) * 4 / 1e9, shape=f"60 s, T={Tf}", device=r"stft_kernel", reps=reps)
+                  gbytes=(x.numel() + src.numel()) * 4 / 1e9, shape=f"60 s, T={Tf}", device=r"[^i]stft(2048)?_kernel", reps=reps)
             mask = torch.randn_like(src)
             out = torch.empty_like(x)
             _emit("istft", _event_time(lambda: model.istft(src, mask, length, out, fm), reps),
                   gbytes=(2 * src.numel() + out.numel()) * 4 / 1e9, shape=f"60 s, T={Tf}",
-                  device=r"istft_frames_kernel|ola_kernel", per_call=2, reps=reps)
+                  device=r"istft(2048)?_frames_kernel|ola_kernel", per_call=2, reps=reps)
             seq = torch.empty(d.bands, Tf, D, device=dev)
             _emit("band_split", _event_time(lambda: model.band_split(src, Tf, seq, fm), reps),
                   gflop=2.0 * Tf * sum(d.input_dims()) * D / 1e9, shape=f"T={Tf}, 62 bands",
-                  device=r"band_gather_norm_kernel|gemm_f32_batched_kernel", per_call=2, reps=reps)
+                  device=r"band_split_kernel", per_call=3, reps=reps)
             feats = torch.randn(Tf, d.bands, D, device=dev, generator=g)
             mout = torch.empty_like(src)
             gf = 2.0 * Tf * (d.bands * D * d.mask_hidden + d.mask_hidden * 2 * sum(d.input_dims())) / 1e9
             r = max(3, reps // 4)
             _emit("mask_estimator", _event_time(lambda: model.mask_estimate(feats, Tf, mout, fm), r),
                   gflop=gf, shape=f"T={Tf}, 62 bands", peak_tflops=FP16_TFLOPS, mc_products=3,
-                  device=r"gemm_h2_batched_kernel|mask_glu_scatter_kernel", per_call=3, reps=r)
+                  device=r"gemm_h2_batched_kernel", per_call=2, reps=r)
         model.close()
     ctx.close()
     return 0

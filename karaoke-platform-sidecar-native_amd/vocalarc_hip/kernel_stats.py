@@ -47,11 +47,13 @@ ROLES = [
     (r"gemm_h2_kernel(<3, false|ILi3ELb0E)",
      "FFN down-projection + residual, raising the stream's bound (fp32 via two-piece fp16)"),
     (r"gemm_h2_kernel(<|ILi)3", "out projection / FFN down-projection + residual (fp32 via two-piece fp16)"),
-    (r"gemm_h2_kernel(<0, false, true[,>]|ILi0ELb0ELb1E)",
+    (r"gemm_h2_kernel(<0, false, .*true, true>|ILi0ELb0E.*ELb1ELb1E)",
      "time-axis fused QKV + gate projection with the attention's pre-norm inside, k (rotated) and v written as the "
      "attention's fp16 pieces (fp32 via two-piece fp16)"),
     (r"gemm_h2_kernel(<|ILi)0", "fused QKV + gate projection (fp32 via two-piece fp16)"),
     (r"gemm_h2_batched_kernel(<|ILi)2", "mask estimator layer 1 + tanh, batched over bands (fp32 via two-piece fp16)"),
+    (r"gemm_h2_batched_kernel(<|ILi)5",
+     "mask estimator layer 2 with the GLU and the bin scatter, batched over bands (fp32 via two-piece fp16)"),
     (r"gemm_h2_batched_kernel(<|ILi)0", "mask estimator layer 2, batched over bands (fp32 via two-piece fp16)"),
     (r"split_weight_h2_kernel", "weight split into fp16 pieces (model load)"),
     (r"scale_columns_kernel", "RMSNorm gain folded into the QKV weight (model load)"),
@@ -80,14 +82,16 @@ ROLES = [
     (r"gemm_bf16_(dma_)?kernel(<|ILi)0", "fused QKV + gate projection (bf16 variant)"),
     (r"gemm_bf16_(dma_)?batched_kernel(<|ILi)2", "mask layer 1 (bf16 variant)"),
     (r"gemm_bf16_(dma_)?batched_kernel(<|ILi)0", "band split / mask layer 2 (bf16 variant)"),
+    (r"attention_bf16_kvp_kernel", "time-axis attention, L = 801, on rotated k (bf16 variant)"),
     (r"attention_bf16_kernel(<|ILi)4", "time-axis attention, L = 801 (bf16 variant)"),
     (r"attention_bf16_kernel(<|ILi)2", "band-axis attention, L = 62 (bf16 variant)"),
     (r"attention_split_kernel", "time-axis attention, L = 801 (fp32 via split bf16)"),
     (r"attention_kernel(<|ILi)4", "time-axis attention, L = 801"),
     (r"attention_short_kernel", "band-axis attention, L = 62"),
     (r"rmsnorm_kernel", "pre-norms and final norm"),
-    (r"istft_frames_kernel", "mask multiply + inverse FFT"),
-    (r"stft_kernel", "STFT"),
+    (r"istft(2048)?_frames_kernel", "mask multiply + inverse FFT"),
+    (r"stft(2048)?_kernel", "STFT"),
+    (r"band_split_kernel", "band split: gather, RMSNorm and linear, one kernel (fp32 via two-piece fp16)"),
     (r"ola_kernel", "overlap-add"),
     (r"band_gather_norm_kernel", "band gather + RMSNorm"),
     (r"mask_glu_scatter_kernel", "mask GLU + bin scatter"),

@@ -169,6 +169,9 @@ DMA_CASES = [
     (1, 8, 32, 0, False),
     (300, 200, 96, 2, True),   # bf16 output leaving through LDS: tanh, ragged last 8-column store
     (70, 5, 32, 0, True),      # fewer columns than one 16-byte store
+    (77600, 384, 32, 3, False),   # blocks of 256 rows, as launches that fill the chip take (128 above)
+    (49662, 384, 64, 3, False),   # 128 rows: 1164 blocks divide over 256 CUs more evenly than 582
+    (50001, 1024, 32, 1, True),   # 256 rows, bf16 output
 ]
 
 

@@ -132,6 +132,35 @@ def test_kv_pieces_consecutive_rows_bit_identical(cfg2_models, rng, monkeypatch,
     assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
 
 
+@pytest.mark.parametrize("axis,S,L", [(0, 3, 129), (1, 5, 160), (0, 2, 801), (0, 31, 191), (0, 0, 0)])
+def test_bf16_rotated_k_bit_identical(cfg2_models, rng, monkeypatch, axis, S, L):
+    """The bf16 variant: k leaves the projection rotated (consecutive rows, and with S = 0 a 2 s forward's
+    [frame][band] rows, 201 frames) and the attention copies k and v into LDS by DMA; the same bits as the rotation
+    and transposition in the attention (VOCALARC_KV_PIECES=0)."""
+    om, dm = cfg2_models
+    x = rng.standard_normal((S, L, om.d.dim), dtype=np.float32) if S else audio.sine_mix(2.0, 15)
+    dm.set_precision(native.PRECISION_BF16)
+    outs = []
+    try:
+        for env in (None, "0"):
+            if env is None:
+                monkeypatch.delenv("VOCALARC_KV_PIECES", raising=False)
+            else:
+                monkeypatch.setenv("VOCALARC_KV_PIECES", env)
+            if S:
+                dx = to_dev(x)
+                dm.transformer(1, axis, dx, S, L)
+            else:
+                dx = empty_dev(x.shape)
+                dm.forward(to_dev(x), x.shape[1], dx)
+            outs.append(from_dev(dx))
+    finally:
+        dm.set_precision(native.PRECISION_FP32)
+        monkeypatch.delenv("VOCALARC_KV_PIECES", raising=False)
+    assert np.all(np.isfinite(outs[0]))
+    assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+
+
 @pytest.mark.parametrize("windows", [1, 3])
 def test_kv_pieces_bit_identical(cfg2_models, monkeypatch, windows):
     """On the pipeline's time axis (L > 64, [chunk][frame][band] rows) the
