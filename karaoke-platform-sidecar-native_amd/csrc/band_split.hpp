@@ -8,7 +8,8 @@
 // Bound by writing the features: 4 D bytes per row and band (571 MB for 60 s at
 // D = 384, against 98 MB read and 57 GFLOP of piece products).  Gathering into
 // memory and a batched fp32 MFMA GEMM took 144 + 367 us for those 6001 rows; this
-// kernel 220 + 47 (the two widest bands).  64 rows, so that a band's pieces (25 KB at the narrowest) are read
+// kernel 260 (44 bands of 8-48 inputs 120, 16 of 96 and 192 98, two of 512
+// and 516 42).  64 rows, so that a band's pieces (25 KB at the narrowest) are read
 // once per 98 KB written; 32 where the rows' 2 KB would not leave two
 // workgroups' worth of LDS.
 //
@@ -43,11 +44,11 @@ struct BandSplitArgs {
     int M, T, C, D;
 };
 
-constexpr int BS_THREADS = 512, BS_BATCH = 4;
+constexpr int BS_BATCH = 4;
 
 // RT rows, KMAX padded inputs at most, J column tiles at a time per wave.
-template <int RT, int KMAX, int J>
-__global__ __launch_bounds__(BS_THREADS, 4) void band_split_kernel(BandSplitArgs a) {
+template <int RT, int KMAX, int J, int BS_THREADS>
+__global__ __launch_bounds__(BS_THREADS, BS_THREADS == 256 ? 3 : 4) void band_split_kernel(BandSplitArgs a) {
     static_assert(RT == 32 || RT == 64, "one or two 32-row blocks");
     constexpr int PARTS = BS_THREADS / RT;
     __shared__ __attribute__((aligned(16))) unsigned char rows[RT * (KMAX * 4 + 16)];
@@ -61,6 +62,36 @@ __global__ __launch_bounds__(BS_THREADS, 4) void band_split_kernel(BandSplitArgs
     const int tid = (int)threadIdx.x;
     const int pitch = d.kpad * 4 + 16;
     const int pairs = d.width * a.C;
+
+    // wave: 32 of the rows and, of the column tiles of 32, every CG-th
+    constexpr int RB = RT / 32, CG = BS_THREADS / 64 / RB;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 31, lh = lane >> 5;
+    const int r0 = 32 * (wave % RB);
+    const int nct = (a.D + 31) / 32, nk = d.kpad / GS_BK;
+    const int eu = -(d.ea + h2_exponent(*static_cast<const float *>(d.W)));
+    const char *const planes = static_cast<const char *>(d.W) + H2_HEADER;
+    const char *wp[J];
+    float bias[J];
+    halfx8 wh[J], wm[J];
+    auto fetch = [&](int k, halfx8 (&h)[J], halfx8 (&m)[J]) {
+#pragma unroll
+        for (int j = 0; j < J; j++) {
+            h[j] = *reinterpret_cast<const halfx8 *>(wp[j] + k * (H2_WBLOCK * 2));
+            m[j] = *reinterpret_cast<const halfx8 *>(wp[j] + k * (H2_WBLOCK * 2) + GS_BN * GS_BK * 2);
+        }
+    };
+    // the column tiles ct0, ct0 + CG, ...: their biases and first pieces
+    auto begin = [&](int ct0) {
+#pragma unroll
+        for (int j = 0; j < J; j++) {
+            const int n = 32 * min(ct0 + CG * j, nct - 1), r = n % GS_BN + li;  // past the last tile: not stored
+            wp[j] = planes + (size_t)(n / GS_BN) * nk * (H2_WBLOCK * 2) + r * 32 + 16 * (lh ^ ((r >> 3) & 1));
+            bias[j] = n + li < a.D ? d.bias[n + li] : 0.0f;
+        }
+        fetch(0, wh, wm);
+    };
+    if (wave / RB < nct) begin(wave / RB);  // on their way while the rows are gathered
 
     // gather: consecutive threads along the spectrum's contiguous direction
     const int ch0 = m0 / a.T, t0 = m0 - ch0 * a.T;
@@ -106,7 +137,6 @@ __global__ __launch_bounds__(BS_THREADS, 4) void band_split_kernel(BandSplitArgs
 
     const int row = tid % RT, pt = tid / RT;
     unsigned char *const rp = rows + row * pitch;
-    const int nk = d.kpad / GS_BK;
     float ss = 0.0f;
     for (int k = pt; k < nk; k += PARTS) {
 #pragma unroll
@@ -143,25 +173,10 @@ __global__ __launch_bounds__(BS_THREADS, 4) void band_split_kernel(BandSplitArgs
     }
     __syncthreads();
 
-    // wave: 32 of the rows and, of the column tiles of 32, every CG-th
-    constexpr int RB = RT / 32, CG = BS_THREADS / 64 / RB;
-    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int li = lane & 31, lh = lane >> 5;
-    const int r0 = 32 * (wave % RB);
-    const int nct = (a.D + 31) / 32;
-    const int eu = -(d.ea + h2_exponent(*static_cast<const float *>(d.W)));
-    const char *const planes = static_cast<const char *>(d.W) + H2_HEADER;
     const unsigned char *const ar = rows + (r0 + li) * pitch + 16 * lh;
     float *const out = a.out + (int64_t)b * a.band_stride + (int64_t)(m0 + r0) * a.ldo;
     for (int ct0 = wave / RB; ct0 < nct; ct0 += CG * J) {
-        const char *wp[J];
-        float bias[J];
-#pragma unroll
-        for (int j = 0; j < J; j++) {
-            const int n = 32 * min(ct0 + CG * j, nct - 1), r = n % GS_BN + li;  // past the last tile: not stored
-            wp[j] = planes + (size_t)(n / GS_BN) * nk * (H2_WBLOCK * 2) + r * 32 + 16 * (lh ^ ((r >> 3) & 1));
-            bias[j] = n + li < a.D ? d.bias[n + li] : 0.0f;
-        }
+        if (ct0 != wave / RB) begin(ct0);
         floatx16 acc[J];
 #pragma unroll
         for (int j = 0; j < J; j++)
@@ -169,15 +184,6 @@ __global__ __launch_bounds__(BS_THREADS, 4) void band_split_kernel(BandSplitArgs
             for (int r = 0; r < 16; r++) acc[j][r] = 0.0f;
         // the pieces of chunk k + 1 are on their way while chunk k is
         // multiplied (the last chunk's are read twice)
-        halfx8 wh[J], wm[J];
-        auto fetch = [&](int k, halfx8 (&h)[J], halfx8 (&m)[J]) {
-#pragma unroll
-            for (int j = 0; j < J; j++) {
-                h[j] = *reinterpret_cast<const halfx8 *>(wp[j] + k * (H2_WBLOCK * 2));
-                m[j] = *reinterpret_cast<const halfx8 *>(wp[j] + k * (H2_WBLOCK * 2) + GS_BN * GS_BK * 2);
-            }
-        };
-        fetch(0, wh, wm);
         for (int k = 0; k < nk; k++) {
             halfx8 nh[J], nm[J];
             fetch(min(k + 1, nk - 1), nh, nm);

@@ -68,7 +68,7 @@ struct vh_model {
     // descriptor, and the bands by the rows' width (band_split_kernel's
     // KMAX); no descriptors: the gather and the fp32 MFMA GEMM run instead
     DeviceBuffer band_pieces, band_descs;
-    std::vector<int> band_class[3];
+    std::vector<int> band_class[4];
     // DSP constants
     DeviceBuffer window, twiddle;
     // pipeline scratch (grown on demand)
@@ -684,7 +684,7 @@ bool prepare_split(vh_model *m) {
 
 // The band split's descriptors: weight pieces and gains padded to K chunks of
 // 16, the exponent of each band's normalised rows.
-constexpr int BAND_CLASS_K[3] = {192, 528, 640};
+constexpr int BAND_CLASSES = 4, BAND_CLASS_K[BAND_CLASSES] = {64, 192, 528, 640};
 bool prepare_band_split(vh_model *m) {
     const Dims &d = m->d;
     hipStream_t s = m->ctx->stream;
@@ -695,7 +695,7 @@ bool prepare_band_split(vh_model *m) {
     for (int b = 0; b < B; b++) {
         total += round(h2_bytes(D, kpad(b))) + round(kpad(b) * sizeof(float));
         widest = std::max(widest, (size_t)D * kpad(b) * sizeof(float));
-        if (kpad(b) > BAND_CLASS_K[2]) return true;
+        if (kpad(b) > BAND_CLASS_K[BAND_CLASSES - 1]) return true;
     }
     DeviceBuffer padded;  // a weight matrix widened to its K chunks
     if (!m->band_pieces.ensure(total, "hipMalloc(band pieces)") || !padded.ensure(widest, "hipMalloc(padded band weight)") ||
@@ -741,7 +741,7 @@ bool prepare_band_split(vh_model *m) {
         if (!(host[2 * b] >= 0.0f && host[2 * b] <= 1.0e30f)) return true;
         descs[b].ea = h2_exponent(host[2 * b]);
     }
-    for (int c = 0; c < 3; c++) {
+    for (int c = 0; c < BAND_CLASSES; c++) {
         for (int b = 0; b < B; b++)
             if (descs[b].kpad <= BAND_CLASS_K[c] && (c == 0 || descs[b].kpad > BAND_CLASS_K[c - 1]))
                 m->band_class[c].push_back(b);
@@ -811,16 +811,17 @@ bool stage_band_split(vh_model *m, const float *source, const SpecLayout &lay, i
         a.ldo = frame_major ? (int64_t)B * D : D;
         a.M = M; a.T = T; a.C = d.channels; a.D = D;
         Scope sc(&m->ctx->timer, s, "gemm_band_split");
-        for (int c = 0; c < 3; c++) {
+        for (int c = 0; c < BAND_CLASSES; c++) {
             a.list = list;
             a.count = (int)m->band_class[c].size();
             list += a.count;
             if (!a.count) continue;
-            const int rt = c == 0 ? 64 : 32;
-            const dim3 grid((unsigned)((M + rt - 1) / rt) * (unsigned)a.count), block(BS_THREADS);
-            if (c == 0) hipLaunchKernelGGL((band_split_kernel<64, BAND_CLASS_K[0], 3>), grid, block, 0, s, a);
-            else if (c == 1) hipLaunchKernelGGL((band_split_kernel<32, BAND_CLASS_K[1], 2>), grid, block, 0, s, a);
-            else hipLaunchKernelGGL((band_split_kernel<32, BAND_CLASS_K[2], 2>), grid, block, 0, s, a);
+            const int rt = c == 1 ? 64 : 32;
+            const dim3 grid((unsigned)((M + rt - 1) / rt) * (unsigned)a.count);
+            if (c == 0) hipLaunchKernelGGL((band_split_kernel<32, BAND_CLASS_K[0], 3, 256>), grid, dim3(256), 0, s, a);
+            else if (c == 1) hipLaunchKernelGGL((band_split_kernel<64, BAND_CLASS_K[1], 3, 512>), grid, dim3(512), 0, s, a);
+            else if (c == 2) hipLaunchKernelGGL((band_split_kernel<32, BAND_CLASS_K[2], 2, 512>), grid, dim3(512), 0, s, a);
+            else hipLaunchKernelGGL((band_split_kernel<32, BAND_CLASS_K[3], 2, 512>), grid, dim3(512), 0, s, a);
             if (!sync_debug(s, "band_split_kernel")) return false;
         }
         return true;
@@ -962,8 +963,8 @@ bool stage_stack(vh_model *m, float *x, int chunks, int T) {
     const Dims &d = m->d;
     const int64_t tokens = (int64_t)chunks * T * d.bands;
     vh_context *ctx = m->ctx;
-    // attention pre-norms fused into the QKV GEMMs: the stream's bound is
-    // found once, then carried from block to block by the FFN-down epilogues
+    // attention pre-norms inside the QKV GEMMs from the second block on: the
+    // stream's bound is raised by each block's FFN-down epilogue for the next
     XBound xb;
     xb.dev = stream_bound(m);
     xb.scratch = absmax_scratch(m);
@@ -1050,8 +1051,8 @@ extern "C" void vh_model_free(vh_model *m) {
 
 extern "C" int vh_transformer(vh_context *ctx, vh_model *m, int layer, int axis, float *x, int S, int L) {
     if (!ctx || !m || layer < 0 || layer >= m->d.depth || axis < 0 || axis > 1 || S <= 0 || L <= 0) return 0;
-    // the attention's pre-norm fused into the QKV GEMM as in the layer stack,
-    // the stream's bound found by an absmax pass (float 8 of the context's bounds)
+    // the stream's bound, for the fused band axis: found by an absmax pass
+    // (float 8 of the context's bounds)
     if (!ctx->bounds.ensure((64 + ABSMAX_PARTIALS) * sizeof(float), "hipMalloc(operand bounds)")) return 0;
     XBound xb;
     xb.dev = ctx->bounds.f() + 8;
