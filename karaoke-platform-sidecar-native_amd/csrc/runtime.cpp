@@ -257,8 +257,9 @@ static void launch_bf16_typed(hipStream_t s, const GemmDescBF16 *single, const G
             if (single) {
                 // 128-row blocks where their finer division of the launch over
                 // the CUs outweighs their 8% higher cost per element (as
-                // h2_tile_pick; N = 384: K = 512 and 1536 at 49662 rows
-                // 104 us each on 256 rows, @@ on 128)
+                // h2_tile_pick).  62 x 20 frames, 1 s and 8 s blocks: 93 -> 85
+                // us at the smallest; N = 384 at 49662 rows (582 blocks of 256
+                // rows, 1164 of 128) 104 -> 104 us
                 auto per_cu = [&](int bm) {
                     const int64_t t = (int64_t)((single->M + bm - 1) / bm) * ((single->N + GBD_BN - 1) / GBD_BN);
                     return (double)((t + device_cus() - 1) / device_cus());
@@ -1221,35 +1222,44 @@ bool transformer_block(hipStream_t s, const Dims &d, const LayerWeights &w, floa
     };
     if (xb && xb->dev && xb->scratch && qkv_h2 && ff1_h2 && w.wqkvg_pg && use_h2(w.wout_p, inner) &&
         use_h2(w.w2_p, d.ff_dim)) {
-        // The attention's pre-norm inside the QKV GEMM (row_norm, the gain in
-        // its pieces), A = x bounded by max |x| in xb->dev: found by an
-        // absmax pass or raised by the previous block's FFN down-projection
-        // epilogue.  The FFN-up GEMM (after the QKV GEMM's last read of the
-        // slot) zeroes it for this block's FFN down-projection to raise.  The
-        // FFN's pre-norm stays a pass of its own: inside the FFN-up GEMM the
-        // split of A, repeated in each of its 24 column tiles, cost more
-        // (+9%) than the pass it saves.
-        if (!xb->valid && !absmax(s, x, tokens * D, xb->scratch, xb->dev)) return false;
-        xb->valid = false;  // until the FFN down-projection has raised the slot
-        GemmArgsH2 gq{x, D, w.wqkvg_pg, w.bqkvg, qkvg, nq, tokens, nq, D};
-        gq.row_norm = true;
-        const bool kv_pre = kv_out(gq), kv_pieces = gq.kv_pieces;
         // On the band axis (sequences of L <= 64 consecutive rows) the
         // projection and the attention run as one kernel (band_attention.hpp):
         // q, k, v and the gate logits stay on chip.  VOCALARC_BAND_FUSED=0
         // keeps the two kernels.
         const char *bf_env = getenv("VOCALARC_BAND_FUSED");
-        const bool band_fused = kv_pre && lay.L <= 64 && lay.group == 1 && lay.seq_stride == 0 &&
-                                lay.pos_stride == 1 && lay.group_stride == lay.L && tokens == (int64_t)lay.S * lay.L &&
-                                D <= BA_MAX_K && inner % GS_BN == 0 && (!d.gated || w.wgate_g) && rt &&
-                                !(bf_env && bf_env[0] == '0');
+        const char *kv_env = getenv("VOCALARC_KV_PRESCALE");
+        const bool band_fused = att_h2 && !(kv_env && kv_env[0] == '0') && lay.L <= 64 && lay.group == 1 &&
+                                lay.seq_stride == 0 && lay.pos_stride == 1 && lay.group_stride == lay.L &&
+                                tokens == (int64_t)lay.S * lay.L && D <= BA_MAX_K && inner % GS_BN == 0 &&
+                                (!d.gated || w.wgate_g) && rt && !(bf_env && bf_env[0] == '0');
+        // The attention's pre-norm inside the QKV GEMM (row_norm, the gain in
+        // its pieces) when the bound of its A, the raw stream x, is there:
+        // max |x| in xb->dev, raised by the previous block's FFN
+        // down-projection epilogue (the FFN-up GEMM, after the last read of
+        // the slot, zeroes it).  A block without one -- the first of a stack, a
+        // block called alone -- runs the norm as a pass instead of an absmax
+        // pass (QKV and what it needs, us: 862 x 90 rows, D = 256: 248 + 19
+        // inside, 231 + 28 as a pass; 62 x 101, D = 384: 33 + 9, 30 + 6);
+        // with the bound at hand inside is the cheaper one (eight windows 1731
+        // against 1570 + 185; 62 x 101: 33 against 30 + 6).  The fused band
+        // axis always takes x and its bound.  The FFN's pre-norm stays a pass:
+        // inside the FFN-up GEMM the split of A, repeated in each of its 24
+        // column tiles, cost more (+9%) than the pass it saves.
+        const bool inside = band_fused || xb->valid;
+        if (!xb->valid && band_fused && !absmax(s, x, tokens * D, xb->scratch, xb->dev)) return false;
+        xb->valid = false;  // until the FFN down-projection has raised the slot
         if (band_fused) {
             BandAttention ba{x, D, D, w.wqkvg_pg, w.bqkvg, d.gated ? w.wgate_g : nullptr,
                              d.gated && w.bqkvg ? w.bqkvg + d.qkv_dim() : nullptr, xb->dev, w.bounds + 1, rt,
                              attn, inner, lay.S, lay.L, d.heads};
             if (!band_attention(s, ba, t)) return false;
         } else {
-            if (!gemm_h2(s, gq, OperandBound{xb->dev, 0.0f}, EPI_STORE, t, "gemm_qkv")) return false;
+            GemmArgsH2 gq{inside ? x : normed, D, inside ? w.wqkvg_pg : w.wqkvg_p, w.bqkvg, qkvg, nq, tokens, nq, D};
+            gq.row_norm = inside;
+            gq.a_h2 = !inside;
+            const bool kv_pre = kv_out(gq), kv_pieces = gq.kv_pieces;
+            if (!inside && !rmsnorm_h2(s, x, D, w.gamma, normed, D, tokens, D, w.bounds, t)) return false;
+            if (!gemm_h2(s, gq, OperandBound{inside ? xb->dev : w.bounds, 0.0f}, EPI_STORE, t, "gemm_qkv")) return false;
             if (!attention(s, qkvg, nq, attn, inner, rt, lay, d.heads, gate, t, false, false, true,
                            att_h2 ? w.bounds + 1 : nullptr, att_h2, kv_pre, false, kv_pieces))
                 return false;

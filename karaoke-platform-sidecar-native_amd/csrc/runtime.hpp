@@ -370,9 +370,10 @@ struct BlockScratch {
 // (sequence, position) to rows.
 // Bound slot of the residual stream x for blocks whose attention pre-norm runs
 // inside the QKV GEMM (gemm_h2 row_norm; its fp32 A is x itself, split by the
-// bound of |x|): *dev bounds x entering a block -- raised by the previous
-// block's FFN-down epilogue, which `valid` records, else found by an absmax
-// pass.  scratch: ABSMAX_PARTIALS device floats.
+// bound of |x|): *dev bounds x entering a block when `valid` -- raised by the
+// previous block's FFN-down epilogue -- else the fused band axis finds it by an
+// absmax pass and other blocks run the norm as a pass.  scratch:
+// ABSMAX_PARTIALS device floats.
 struct XBound {
     float *dev = nullptr;
     float *scratch = nullptr;
@@ -380,8 +381,8 @@ struct XBound {
 };
 // One pre-norm transformer block on x in place.  With xb (and the gain-folded
 // QKV pieces in w, every linear on the fp16 pieces) the attention's pre-norm
-// is fused into the QKV GEMM; otherwise the RMSNorm kernel writes the
-// normalised rows for both.
+// runs inside the QKV GEMM or the fused band-axis kernel where x's bound is at
+// hand; otherwise the RMSNorm kernel writes the normalised rows for both.
 bool transformer_block(hipStream_t s, const Dims &d, const LayerWeights &w, float *x, int64_t tokens,
                        const AttnLayout &lay, BlockScratch &scr, RopeCache &rope, KernelTimer *t = nullptr,
                        int precision = PREC_FP32, XBound *xb = nullptr);
