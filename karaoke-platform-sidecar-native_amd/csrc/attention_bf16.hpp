@@ -180,9 +180,9 @@ __global__ __launch_bounds__(64 * WAVES, 4) void attention_bf16_kernel(AttnArgs 
 // ds_read_b64_tr_b16, swizzles and read orders as attention_h2_kvp_kernel's, the
 // key blocks' pipeline too.  The register-staged kernel rotates every key once
 // per 128 queries and transposes V by 2-byte LDS writes: 62 x 801 x 8 heads
-// 220 us, this kernel @@ (with the rotation in the projection: @@ -> @@).  Bound
-// by the softmax's VALU work (some 110 instructions beside 8 MFMAs per wave
-// and block).  Same bits as attention_bf16_kernel.
+// 220 us, this kernel 158.  Bound by the softmax's VALU work (some 110
+// instructions beside 8 MFMAs per wave and block).  Same bits as
+// attention_bf16_kernel.
 constexpr int KVB_ROW = 128;                 // bytes of a key's 64 dims
 constexpr int KVB_TILE = ATT_KB * KVB_ROW;   // 4 KB
 template <typename TO>

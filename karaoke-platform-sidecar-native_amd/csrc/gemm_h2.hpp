@@ -565,16 +565,32 @@ __global__ __launch_bounds__(T::THREADS, T::OCC) void gemm_h2_kernel(GemmDescH2 
 }
 
 // Ragged batch (the mask estimator's per-band linears): problem blockIdx.z,
-// one bound for all problems.
+// one bound for all problems; as kernel arguments, 64 bytes each, so that both
+// models' bands fit one launch (the 90-band model's second launch waited for
+// the whole of the first: its mask on 1 s 108 -> 77 us).
+constexpr int H2_MAX_BATCH = 96;
+struct GemmBatchItemH2 {
+    const float *A;
+    const void *W;
+    const float *bias;
+    float *C;
+    int M, N, K, lda, ldc;
+    int mask_f0, mask_dim;  // EPI_MASK_GLU
+};
 struct GemmBatchH2 {
-    GemmDescH2 d[GS_MAX_BATCH];
+    GemmBatchItemH2 d[H2_MAX_BATCH];
     H2Bound b;
     H2MaskOut mo;  // EPI_MASK_GLU
 };
 
 template <int EPI, class T>
 __global__ __launch_bounds__(T::THREADS, T::OCC) void gemm_h2_batched_kernel(GemmBatchH2 b) {
-    gemm_h2_body<EPI, false, T>(b.d[blockIdx.z], b.b.ptr ? *b.b.ptr : b.b.value, (int)blockIdx.x, &b.mo);
+    const GemmBatchItemH2 &i = b.d[blockIdx.z];
+    GemmDescH2 d{};
+    d.A = i.A; d.W = i.W; d.bias = i.bias; d.C = i.C;
+    d.M = i.M; d.N = i.N; d.K = i.K; d.lda = i.lda; d.ldc = i.ldc;
+    d.mask_f0 = i.mask_f0; d.mask_dim = i.mask_dim;
+    gemm_h2_body<EPI, false, T>(d, b.b.ptr ? *b.b.ptr : b.b.value, (int)blockIdx.x, &b.mo);
 }
 
 // max |W| over W [N][ldw] (first K columns) into out[0]; one workgroup of

@@ -220,11 +220,6 @@ __global__ __launch_bounds__(GS_THREADS, 2) void gemm_split_kernel(GemmDescSplit
     gemm_split_body<EPI>(d, xcd_swizzle((int)blockIdx.x, (int)gridDim.x));
 }
 
-// Problems per launch of the ragged batched GEMMs (the mask estimator's
-// per-band linears): descriptors in the kernel arguments, problem blockIdx.z,
-// blocks past a problem's tiles return.
-constexpr int GS_MAX_BATCH = 64;
-
 // fp32 W [N][ldw_in] (K a multiple of 16) -> its h, m, l pieces, tile-major:
 // element (n, k) of piece p at
 //   ((n/128 * K/16 + k/16) * 3 + p) * 2048 + (n%128) * 16 + 8 * (s ^ (n/8)%2) + e

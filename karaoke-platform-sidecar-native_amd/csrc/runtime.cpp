@@ -257,9 +257,9 @@ static void launch_bf16_typed(hipStream_t s, const GemmDescBF16 *single, const G
             if (single) {
                 // 128-row blocks where their finer division of the launch over
                 // the CUs outweighs their 8% higher cost per element (as
-                // h2_tile_pick).  62 x 20 frames, 1 s and 8 s blocks: 93 -> 85
-                // us at the smallest; N = 384 at 49662 rows (582 blocks of 256
-                // rows, 1164 of 128) 104 -> 104 us
+                // h2_tile_pick): a block of few frames 93 -> 85 us, N = 384
+                // at 49662 rows (582 blocks of 256 rows, 1164 of 128) 104 us
+                // either way
                 auto per_cu = [&](int bm) {
                     const int64_t t = (int64_t)((single->M + bm - 1) / bm) * ((single->N + GBD_BN - 1) / GBD_BN);
                     return (double)((t + device_cus() - 1) / device_cus());
@@ -608,8 +608,8 @@ static void launch_h2_batched(hipStream_t s, const GemmBatchH2 &b, unsigned n) {
 bool gemm_h2_batched(hipStream_t s, const std::vector<GemmArgsH2> &gs, const OperandBound &bound, int epilogue,
                      KernelTimer *t, const char *name) {
     Scope sc(t, s, name);
-    for (size_t first = 0; first < gs.size(); first += GS_MAX_BATCH) {
-        const size_t count = std::min(gs.size() - first, (size_t)GS_MAX_BATCH);
+    for (size_t first = 0; first < gs.size(); first += H2_MAX_BATCH) {
+        const size_t count = std::min(gs.size() - first, (size_t)H2_MAX_BATCH);
         GemmBatchH2 b;
         memset(&b, 0, sizeof(b));
         b.b = H2Bound{bound.dev, bound.value};
@@ -626,7 +626,7 @@ bool gemm_h2_batched(hipStream_t s, const std::vector<GemmArgsH2> &gs, const Ope
                 set_error("gemm_h2_batched: row_norm, a_h2, kv_inner, zero_slot and amax are not supported");
                 return false;
             }
-            b.d[i] = to_desc_h2(g);
+            b.d[i] = {g.A, g.W, g.bias, g.C, (int)g.M, g.N, g.K, g.lda, g.ldc, 0, 0};
         }
         const unsigned n = (unsigned)count;
         switch (epilogue) {
@@ -645,8 +645,8 @@ bool gemm_h2_batched(hipStream_t s, const std::vector<GemmArgsH2> &gs, const Ope
 bool gemm_h2_mask(hipStream_t s, const std::vector<MaskBandH2> &bands, int64_t M, const OperandBound &bound, float *mask,
                   const SpecLayout &lay, int T, int C, KernelTimer *t, const char *name) {
     Scope sc(t, s, name);
-    for (size_t first = 0; first < bands.size(); first += GS_MAX_BATCH) {
-        const size_t count = std::min(bands.size() - first, (size_t)GS_MAX_BATCH);
+    for (size_t first = 0; first < bands.size(); first += H2_MAX_BATCH) {
+        const size_t count = std::min(bands.size() - first, (size_t)H2_MAX_BATCH);
         GemmBatchH2 b;
         memset(&b, 0, sizeof(b));
         b.b = H2Bound{bound.dev, bound.value};
@@ -658,9 +658,7 @@ bool gemm_h2_mask(hipStream_t s, const std::vector<MaskBandH2> &bands, int64_t M
                 set_error("gemm_h2_mask: unsupported shape M=%lld dim=%d K=%d lda=%d", (long long)M, m.dim, m.K, m.lda);
                 return false;
             }
-            b.d[i] = to_desc_h2(g);
-            b.d[i].mask_f0 = m.first_freq;
-            b.d[i].mask_dim = m.dim;
+            b.d[i] = {g.A, g.W, g.bias, g.C, (int)g.M, g.N, g.K, g.lda, g.ldc, m.first_freq, m.dim};
         }
         launch_h2_batched<EPI_MASK_GLU>(s, b, (unsigned)count);
         if (!sync_debug(s, "gemm_h2_batched_kernel (mask)")) return false;
