@@ -145,12 +145,12 @@ def test_resident_path_matches_oracle(provider, views, ref_pack):
 
 
 @pytest.mark.parametrize("bands,T", [(90, 47), (130, 31), (130, 47), (161, 129)])
-def test_resident_band_axis_matches_consecutive_rows(provider, views, rng, bands, T):
+def test_resident_band_axis_matches_consecutive_rows(provider, views, bands, T):
     """The band axis of the resident [band][frame] tensor is read in place: its keys' rotary position is row / T
     (more than 128 bands and T >= 32: k leaves the projection rotated and split; else the attention does it).  The
     same block on the transposed tensor (consecutive rows) gives the same bits."""
     L, g = provider
-    x = rng.standard_normal((bands, T, RD.dim), dtype=np.float32)
+    x = np.random.default_rng(T).standard_normal((bands, T, RD.dim), dtype=np.float32)
     w = _weights(views, 0, 1)
     got = np.empty((T, bands, RD.dim), np.float32)
     assert L.native_gpu_resident_begin(g, bands, T, x.ctypes.data) == 1

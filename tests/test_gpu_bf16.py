@@ -169,9 +169,6 @@ DMA_CASES = [
     (1, 8, 32, 0, False),
     (300, 200, 96, 2, True),   # bf16 output leaving through LDS: tanh, ragged last 8-column store
     (70, 5, 32, 0, True),      # fewer columns than one 16-byte store
-    (77600, 384, 32, 3, False),   # blocks of 256 rows, as launches that fill the chip take (128 above)
-    (49662, 384, 64, 3, False),   # 128 rows: 1164 blocks divide over 256 CUs more evenly than 582
-    (50001, 1024, 32, 1, True),   # 256 rows, bf16 output
 ]
 
 
@@ -200,6 +197,16 @@ def test_gemm_bf16_dma_matches_staged(ctx, rng, M, N, K, epi, c16):
     if epi == native.EPI_STORE and not c16:
         assert_close(ref.astype(np.float32), from_dev(outs[0]), rtol=1e-5, atol=1e-5 * (np.sqrt(K) * 0.2 + 1),
                      what="dma gemm")
+
+
+@pytest.mark.parametrize("M,N,K,epi,c16", [
+    (77600, 384, 32, 3, False),   # blocks of 256 rows, as launches that fill the chip take (128 above)
+    (49662, 384, 64, 3, False),   # 128 rows: 1164 blocks divide over 256 CUs more evenly than 582
+    (50001, 1024, 32, 1, True),   # 256 rows, bf16 output
+])
+def test_gemm_bf16_dma_blocks_match_staged(ctx, M, N, K, epi, c16):
+    """The DMA ring's two block heights on launches of many blocks: the register-staged kernel's bits."""
+    test_gemm_bf16_dma_matches_staged(ctx, np.random.default_rng(N), M, N, K, epi, c16)
 
 
 def test_gemm_bf16_operand_alignment_checks(ctx):

@@ -113,10 +113,11 @@ def test_band_attention_fused(cfg2_models, rng, monkeypatch, S, L):
 
 
 @pytest.mark.parametrize("axis,S,L", [(0, 3, 129), (1, 5, 160), (0, 2, 801), (0, 31, 191)])
-def test_kv_pieces_consecutive_rows_bit_identical(cfg2_models, rng, monkeypatch, axis, S, L):
+def test_kv_pieces_consecutive_rows_bit_identical(cfg2_models, monkeypatch, axis, S, L):
     """A block on sequences of consecutive rows (vh_transformer's order): the QKV GEMM rotates k by one position
     per row, sequences ending inside a wave's 32 rows, and a ragged last row tile; the same bits as the attention's own
     rotation and split (VOCALARC_KV_PIECES=0)."""
+    rng = np.random.default_rng(L)
     om, dm = cfg2_models
     x = rng.standard_normal((S, L, om.d.dim), dtype=np.float32)
     outs = []
@@ -133,10 +134,11 @@ def test_kv_pieces_consecutive_rows_bit_identical(cfg2_models, rng, monkeypatch,
 
 
 @pytest.mark.parametrize("axis,S,L", [(0, 3, 129), (1, 5, 160), (0, 2, 801), (0, 31, 191), (0, 0, 0)])
-def test_bf16_rotated_k_bit_identical(cfg2_models, rng, monkeypatch, axis, S, L):
+def test_bf16_rotated_k_bit_identical(cfg2_models, monkeypatch, axis, S, L):
     """The bf16 variant: k leaves the projection rotated (consecutive rows, and with S = 0 a 2 s forward's
     [frame][band] rows, 201 frames) and the attention copies k and v into LDS by DMA; the same bits as the rotation
     and transposition in the attention (VOCALARC_KV_PIECES=0)."""
+    rng = np.random.default_rng(L)
     om, dm = cfg2_models
     x = rng.standard_normal((S, L, om.d.dim), dtype=np.float32) if S else audio.sine_mix(2.0, 15)
     dm.set_precision(native.PRECISION_BF16)
@@ -239,10 +241,11 @@ def test_stft_istft(ctx, cfg2_models, ref_models, which, layout):
 
 @pytest.mark.parametrize("layout", LAYOUTS)
 @pytest.mark.parametrize("length", [1200, 2049, 3969, 4410])
-def test_stft_istft_edges(cfg2_models, rng, length, layout):
+def test_stft_istft_edges(cfg2_models, length, layout):
     """Signals of a few frames (3, 5, 9 or 11: the kernels take four at a time), reflected at both ends, digital
     silence in the first half of one channel, and a mask that makes bins 0 and 1024 complex (only their real parts
     reach the signal)."""
+    rng = np.random.default_rng(length)
     om, dm = cfg2_models
     d = om.d
     x = rng.standard_normal((d.channels, length)).astype(np.float32)
@@ -300,10 +303,11 @@ def test_band_split_and_mask(ctx, cfg2_models, ref_models, which, rng, layout):
 @pytest.mark.parametrize("layout", LAYOUTS)
 @pytest.mark.parametrize("T", [1, 31, 33, 65, 130])
 @pytest.mark.parametrize("which", ["config", "reference"])
-def test_band_split_and_mask_row_tiles(cfg2_models, ref_models, which, rng, T, layout):
+def test_band_split_and_mask_row_tiles(cfg2_models, ref_models, which, T, layout):
     """Frames around the kernels' 32 and 64 row tiles, of very different level (the rows are normalised before
     they are split into fp16 pieces, so quiet frames keep their precision) and one of zeros; the mask's GLU and
     scatter on ragged row tiles, bands of 8 to 516 inputs (16-wide value and gate groups)."""
+    rng = np.random.default_rng(T)
     om, dm = cfg2_models if which == "config" else ref_models
     d = om.d
     src = rng.standard_normal((d.freq_bins, d.channels, T, 2)).astype(np.float32)
@@ -318,6 +322,21 @@ def test_band_split_and_mask_row_tiles(cfg2_models, ref_models, which, rng, T, l
     dmask = empty_dev(_to_layout(mref, layout).shape)
     dm.mask_estimate(to_dev(feats), T, dmask, layout)
     assert_close(mref, _from_layout(from_dev(dmask), layout), rtol=1e-4, atol=1e-5, min_snr=110, what="mask")
+
+
+def test_short_windows_share_row_tiles(cfg2_models):
+    """Windows of 11 frames, up to nine in a pass: a row tile of the band split and of the mask's second layer, and a
+    wave of the projection, span several windows.  Against the same windows one at a time: the values differ only by
+    the operand scales, which follow the pass's largest value."""
+    om, dm = cfg2_models
+    x = audio.sine_mix(0.5, 21)
+    length, chunk, step = x.shape[1], 4410, 2205
+    outs = []
+    for batch in (9, 1):
+        dv = empty_dev(x.shape)
+        dm.separate(to_dev(x), length, chunk, step, batch, dv)
+        outs.append(from_dev(dv))
+    assert_close(outs[1], outs[0], rtol=1e-4, atol=1e-6, min_snr=110, what="windows together")
 
 
 def test_forward_config_shape(cfg2_models):
