@@ -44,10 +44,10 @@ struct BandSplitArgs {
     int M, T, C, D;
 };
 
-constexpr int BS_BATCH = 4;
-
-// RT rows, KMAX padded inputs at most, J column tiles at a time per wave.
-template <int RT, int KMAX, int J, int BS_THREADS>
+// RT rows, KMAX padded inputs at most, J column tiles at a time per wave,
+// BS_BATCH gather loads in flight per thread (enough for a tile's bins at once
+// up to 528 inputs: a tile waits on memory once).
+template <int RT, int KMAX, int J, int BS_THREADS, int BS_BATCH>
 __global__ __launch_bounds__(BS_THREADS, BS_THREADS == 256 ? 3 : 4) void band_split_kernel(BandSplitArgs a) {
     static_assert(RT == 32 || RT == 64, "one or two 32-row blocks");
     constexpr int PARTS = BS_THREADS / RT;

@@ -818,10 +818,10 @@ bool stage_band_split(vh_model *m, const float *source, const SpecLayout &lay, i
             if (!a.count) continue;
             const int rt = c == 1 ? 64 : 32;
             const dim3 grid((unsigned)((M + rt - 1) / rt) * (unsigned)a.count);
-            if (c == 0) hipLaunchKernelGGL((band_split_kernel<32, BAND_CLASS_K[0], 3, 256>), grid, dim3(256), 0, s, a);
-            else if (c == 1) hipLaunchKernelGGL((band_split_kernel<64, BAND_CLASS_K[1], 3, 512>), grid, dim3(512), 0, s, a);
-            else if (c == 2) hipLaunchKernelGGL((band_split_kernel<32, BAND_CLASS_K[2], 2, 512>), grid, dim3(512), 0, s, a);
-            else hipLaunchKernelGGL((band_split_kernel<32, BAND_CLASS_K[3], 2, 512>), grid, dim3(512), 0, s, a);
+            if (c == 0) hipLaunchKernelGGL((band_split_kernel<32, BAND_CLASS_K[0], 3, 256, 4>), grid, dim3(256), 0, s, a);
+            else if (c == 1) hipLaunchKernelGGL((band_split_kernel<64, BAND_CLASS_K[1], 3, 512, 12>), grid, dim3(512), 0, s, a);
+            else if (c == 2) hipLaunchKernelGGL((band_split_kernel<32, BAND_CLASS_K[2], 2, 512, 17>), grid, dim3(512), 0, s, a);
+            else hipLaunchKernelGGL((band_split_kernel<32, BAND_CLASS_K[3], 2, 512, 10>), grid, dim3(512), 0, s, a);
             if (!sync_debug(s, "band_split_kernel")) return false;
         }
         return true;
