@@ -7,7 +7,7 @@ depth 12, 62 bands, 8 heads x 64, GELU-GLU FFN (mult 4), hop 441, n_fft 2048:
 8 s windows with 2 s overlap (50 windows), 8 windows per device pass, linear
 cross-fade.  The input waveform is resident in HBM when the timed region
 starts; the output waveform is in HBM when it ends.  fp32 accuracy for
-`value`: the transformer and mask-estimator linears and the attention
+`value`: the transformer, band-split and mask-estimator linears and the attention
 products of both axes run on the fp16 matrix cores as two-piece splits of
 their power-of-two-scaled fp32 operands (three piece products per fp32
 product, fp32 accumulation), everything else on fp32 MFMA / fp32 / fp64.
@@ -428,10 +428,10 @@ def main() -> int:
         "scaling": "weak",
         "vs_baseline": None,
         "dtype": "fp32",
-        "precision_note": "fp32 accuracy: transformer and mask-estimator linears as 2-piece fp16 splits of "
+        "precision_note": "fp32 accuracy: transformer, band-split and mask-estimator linears as 2-piece fp16 splits of "
                           "power-of-two-scaled operands (3 products, fp32 accumulation; error vs fp64 at or below "
                           "the fp32 MFMA GEMM's), time- and band-axis attention the same way (bound from the "
-                          "QKV projection's weights), band split on fp32 MFMA, DSP in fp64/fp32",
+                          "QKV projection's weights), DSP in fp64/fp32",
         "data": "synthetic (seeded sine+noise mix, random-init weights N(0,0.02), gammas N(1,0.02))",
         "config": {
             "workload": "full BS-RoFormer separation, 5 min stereo 44.1 kHz, 8 s windows / 2 s overlap, "

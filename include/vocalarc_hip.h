@@ -202,13 +202,12 @@ void vh_model_free(vh_model *model);
 /* Arithmetic of the model's matrix products (every linear of the transformer
    stack, band split and mask estimator):
    VH_PRECISION_FP32 (default, the parity path): fp32 accuracy.  The
-     transformer and mask-estimator linears run on fp16 matrix cores by
+     transformer, band-split and mask-estimator linears run on fp16 matrix cores by
      two-piece operand splitting (vh_gemm_h2; pieces and operand bounds made
      at load), and so does the attention on both axes (the two-piece
      kernels of VH_ATT_H2, scaled from the fused projection's weight bound;
      a layer whose bound lies outside their scale range runs its attention
-     on the kernels without piece scales); the band split runs on the fp32
-     MFMA instruction.
+     on the kernels without piece scales).
    VH_PRECISION_FP32_MFMA: every product on the fp32 MFMA instruction.
    VH_PRECISION_BF16: activations rounded to bf16 as they enter the matrix
      cores, bf16 weight copies made on the first switch, fp32 accumulation,
