@@ -45,6 +45,12 @@ typedef struct vh_model vh_model;
 vh_context *vh_create(void);
 /* Also frees every model loaded in ctx that vh_model_free has not freed. */
 void vh_destroy(vh_context *ctx);
+/* Later calls issue their work on hip_stream, after all that the context has
+   issued on its earlier streams (its scratch is shared): the new stream waits
+   for an event recorded on the old one, the host does not.  No order is made
+   into or out of a stream that is capturing; the next switch between streams
+   that are not makes it up.  A stream with work that vh_synchronize has not
+   completed may be destroyed only after the switch away from it. */
 int vh_set_stream(vh_context *ctx, void *hip_stream);
 int vh_synchronize(vh_context *ctx);
 const char *vh_last_error(void);

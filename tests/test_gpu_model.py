@@ -13,6 +13,7 @@ from helpers import assert_close, empty_dev, from_dev, gpu_available, snr_db, to
 pytestmark = pytest.mark.gpu
 
 if gpu_available():
+    import torch
     import oracle as O
     from vocalarc_hip import audio, native, pack
     from vocalarc_hip.dims import CONFIG_DIMS, REFERENCE_DIMS
@@ -322,6 +323,48 @@ def test_band_split_and_mask_row_tiles(cfg2_models, ref_models, which, T, layout
     dmask = empty_dev(_to_layout(mref, layout).shape)
     dm.mask_estimate(to_dev(feats), T, dmask, layout)
     assert_close(mref, _from_layout(from_dev(dmask), layout), rtol=1e-4, atol=1e-5, min_snr=110, what="mask")
+
+
+@pytest.mark.parametrize("precision", [0, 1, 2])
+def test_stream_switch_keeps_order(ctx, cfg2_models, precision):
+    """A context's calls share its scratch, so a new stream waits for the work issued on the old one: the end of a call
+    on B implies that of a long one on A, and mask estimates issued in turn on two streams give what they give on one."""
+    om, dm = cfg2_models
+    d, T = om.d, 301
+    g = torch.Generator("cuda:0").manual_seed(31 + precision)
+    feats = [torch.randn(T, d.bands, d.dim, device="cuda:0", generator=g) * s for s in (1.0, 3.0, 0.1, 2.0)]
+    shape = (d.freq_bins, d.channels, T, 2)
+    big, small = torch.randn(8192, 8192, device="cuda:0", generator=g), torch.zeros(64, device="cuda:0")
+    home = torch.cuda.current_stream().cuda_stream
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    dm.set_precision(precision)
+    try:
+        want = []
+        for f in feats:
+            want.append(empty_dev(shape))
+            dm.mask_estimate(f, T, want[-1])
+        torch.cuda.synchronize()
+        ctx.set_stream(a.cuda_stream)
+        with torch.cuda.stream(a):
+            for _ in range(4):
+                big @ big
+        ctx.residual_add(small, small, 32)
+        done = a.record_event()
+        ctx.set_stream(b.cuda_stream)
+        ctx.residual_add(small[32:], small[32:], 32)
+        b.synchronize()
+        assert done.query()  # B's call ended after A's
+        got = [empty_dev(shape) for _ in feats]
+        torch.cuda.synchronize()
+        for i, (f, o) in enumerate(zip(feats, got)):
+            ctx.set_stream((a, b)[i % 2].cuda_stream)
+            dm.mask_estimate(f, T, o)
+        torch.cuda.synchronize()
+    finally:
+        ctx.set_stream(home)
+        dm.set_precision(native.PRECISION_FP32)
+    for w, o in zip(want, got):
+        assert torch.equal(w, o)
 
 
 def test_short_windows_share_row_tiles(cfg2_models):
