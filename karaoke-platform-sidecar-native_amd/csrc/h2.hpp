@@ -31,6 +31,11 @@ VH_HOST_DEVICE inline int h2_exponent(float bound) {
     return e < -100 ? -100 : (e > 100 ? 100 : e);
 }
 
+// Whether h2_exponent of this bound is not clamped (0: all elements are): below
+// the range the pieces of the largest elements lose bits, above it they
+// overflow.
+inline bool h2_exponent_in_range(float bound) { return bound == 0.0f || (bound >= 0x1p-87f && bound < 0x1p114f); }
+
 // Bounds for which the fp16 two-piece attention kernels may run.  They undo
 // the q and k scales with the single power of two 2^-(ek + eq), and the
 // output's with 2^-(ev + 5); with B in [2^-40, 2^60] every exponent lies in

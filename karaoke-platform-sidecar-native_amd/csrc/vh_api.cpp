@@ -737,7 +737,7 @@ bool prepare_band_split(vh_model *m) {
     const int B = d.bands, D = d.dim;
     auto kpad = [&](int b) { return (d.in_dim(b) + GS_BK - 1) / GS_BK * GS_BK; };
     auto round = [](size_t n) { return (n + 255) & ~(size_t)255; };
-    size_t total = round(2 * (size_t)B * sizeof(float)), widest = 0;
+    size_t total = round(3 * (size_t)B * sizeof(float)), widest = 0;
     for (int b = 0; b < B; b++) {
         total += round(h2_bytes(D, kpad(b))) + round(kpad(b) * sizeof(float));
         widest = std::max(widest, (size_t)D * kpad(b) * sizeof(float));
@@ -748,8 +748,8 @@ bool prepare_band_split(vh_model *m) {
         !check(hipMemsetAsync(m->band_pieces.ptr, 0, total, s), "hipMemset(band pieces)"))
         return false;
     char *cur = static_cast<char *>(m->band_pieces.ptr);
-    float *bounds = reinterpret_cast<float *>(cur);
-    cur += round(2 * (size_t)B * sizeof(float));
+    float *bounds = reinterpret_cast<float *>(cur);  // two per band, then max |W| of each
+    cur += round(3 * (size_t)B * sizeof(float));
     std::vector<BandSplitDesc> descs(B);
     for (int b = 0; b < B; b++) {
         const int K = d.in_dim(b), P = kpad(b);
@@ -763,7 +763,9 @@ bool prepare_band_split(vh_model *m) {
                 return false;
             W = padded.f();
         }
-        if (!split_weights_h2(s, W, D, P, P, cur)) return false;
+        if (!split_weights_h2(s, W, D, P, P, cur) ||
+            !check(hipMemcpyAsync(bounds + 2 * B + b, cur, sizeof(float), hipMemcpyDeviceToDevice, s), "hipMemcpy(max |W|)"))
+            return false;
         cur += round(h2_bytes(D, P));
         e.gamma = reinterpret_cast<float *>(cur);
         if (!check(hipMemcpyAsync(cur, m->band_gamma[b], K * sizeof(float), hipMemcpyDeviceToDevice, s),
@@ -776,15 +778,18 @@ bool prepare_band_split(vh_model *m) {
         e.kpad = P;
         if (!operand_bounds(s, m->band_gamma[b], K, nullptr, 0, nullptr, false, bounds + 2 * b)) return false;
     }
-    std::vector<float> host(2 * (size_t)B);
+    std::vector<float> host(3 * (size_t)B);
     if (!check(hipMemcpyAsync(host.data(), bounds, host.size() * sizeof(float), hipMemcpyDeviceToHost, s),
                "hipMemcpy(band bounds)") ||
         !check(hipStreamSynchronize(s), "hipStreamSynchronize(band bounds)"))
         return false;
     std::vector<int> list;
     for (int b = 0; b < B; b++) {
-        // beyond the scale range: the band split stays on fp32 MFMA
-        if (!(host[2 * b] >= 0.0f && host[2 * b] <= 1.0e30f)) return true;
+        // gains or weights beyond the scale range: the band split stays on fp32 MFMA
+        if (!h2_exponent_in_range(host[2 * b]) || !h2_exponent_in_range(host[2 * B + b])) {
+            m->band_pieces.release();
+            return true;
+        }
         descs[b].ea = h2_exponent(host[2 * b]);
     }
     for (int c = 0; c < BAND_CLASSES; c++) {

@@ -325,6 +325,27 @@ def test_band_split_and_mask_row_tiles(cfg2_models, ref_models, which, T, layout
     assert_close(mref, _from_layout(from_dev(dmask), layout), rtol=1e-4, atol=1e-5, min_snr=110, what="mask")
 
 
+@pytest.mark.parametrize("name,power", [("weight", 121), ("weight", -110), ("gamma", 118), ("gamma", -118)])
+def test_band_split_outside_scale_range(ctx, name, power):
+    """One band's weights or gains so large or so small that their power-of-two scale would be clamped: the fp16 pieces
+    would overflow or lose bits, so the band split runs on the fp32 MFMA instruction."""
+    d = CONFIG_DIMS.with_depth(0)
+    blob = pack.synthetic_pack(d, 78)
+    views = pack.tensor_views(d, blob)
+    band = 50  # 96 inputs
+    views[f"bands.{band}.{name}"] *= np.float32(2.0 ** power)
+    views[f"bands.{band}.bias"] *= 0
+    src = np.random.default_rng(9).standard_normal((d.freq_bins, d.channels, 40, 2)).astype(np.float32)
+    ref = O.Model(d, blob).band_split(src)
+    dm = native.Model(ctx, d, blob)
+    dout = empty_dev(ref.shape)
+    dm.band_split(to_dev(src), 40, dout)
+    out = from_dev(dout)
+    dm.close()
+    scale = np.abs(ref).max(axis=(1, 2), keepdims=True).astype(np.float64)
+    assert_close(ref / scale, out / scale, rtol=1e-4, atol=2e-5, min_snr=110, what="band split")
+
+
 @pytest.mark.parametrize("precision", [0, 1, 2])
 def test_stream_switch_keeps_order(ctx, cfg2_models, precision):
     """A context's calls share its scratch, so a new stream waits for the work issued on the old one: the end of a call
