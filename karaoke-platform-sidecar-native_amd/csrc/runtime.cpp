@@ -249,22 +249,34 @@ static bool dma_ok(const GemmArgsBF16 &g) {
     return g.a_bf16 && g.K % GBD_BK == 0 && !g.staged && g.lda <= (1 << 21) && g.ldb <= (1 << 21);
 }
 
+// Whether the DMA kernel takes 128-row blocks: where their finer division of
+// the launch over the CUs outweighs their 8% higher cost per element (us on
+// 128 and 256 rows: N = 384, K = 1536 at 3968 rows 19.5 and 26.4, at 49662 92.6
+// and 96.0; K = 512 there 52.0 and 56.1; N = 3072, K = 384 at 6262 rows 23.7 and
+// 26.0).  Not past three 256-row blocks per CU at K > 512, five for the
+// residual epilogue: there the weights and C's fp32 rows, not the division, are
+// the time (N = 256, K = 1024 at 99262 rows, four per CU: 107.5 and 93.1; N = 384,
+// K = 1536 at 115000, six: 238 and 222; N = 256, K = 512 at 180000, six: 127 and
+// 119), while bf16 outputs of short K still gain (N = 1024, K = 256 at 43000, six:
+// 45 and 48).  Both models' linears at 24 row counts from 1240 to 397296: within
+// 1.2% of the better height on average.
+static bool bf16_rows128(const GemmDescBF16 &d, bool residual) {
+    auto per_cu = [&](int bm) {
+        const int64_t t = (int64_t)((d.M + bm - 1) / bm) * ((d.N + GBD_BN - 1) / GBD_BN);
+        return (t + device_cus() - 1) / device_cus();
+    };
+    const int64_t full = per_cu(256);
+    if (full > (d.K > 512 ? 3 : residual ? 5 : INT32_MAX)) return false;
+    return std::max((double)per_cu(128) * 1.08, 1.47) < (double)full * 2.0;
+}
+
 template <int EPI, typename TA, typename TC>
 static void launch_bf16_typed(hipStream_t s, const GemmDescBF16 *single, const GemmBatchBF16 *batch, unsigned tiles,
                               unsigned n, bool dma) {
     if constexpr (std::is_same<TA, bf16>::value) {
         if (dma) {
             if (single) {
-                // 128-row blocks where their finer division of the launch over
-                // the CUs outweighs their 8% higher cost per element (as
-                // h2_tile_pick): a block of few frames 93 -> 85 us, N = 384
-                // at 49662 rows (582 blocks of 256 rows, 1164 of 128) 104 us
-                // either way
-                auto per_cu = [&](int bm) {
-                    const int64_t t = (int64_t)((single->M + bm - 1) / bm) * ((single->N + GBD_BN - 1) / GBD_BN);
-                    return (double)((t + device_cus() - 1) / device_cus());
-                };
-                if (std::max(per_cu(128) * 1.08, 1.47) < per_cu(256) * 2.0)
+                if (bf16_rows128(*single, EPI == EPI_RESIDUAL))
                     hipLaunchKernelGGL((gemm_bf16_dma_kernel<EPI, TC, 2>),
                                        dim3((unsigned)((single->M + 127) / 128) * (unsigned)((single->N + GBD_BN - 1) / GBD_BN)),
                                        dim3(256), 0, s, *single);
