@@ -198,8 +198,10 @@ bool gemm_batched(hipStream_t s, const std::vector<GemmArgs> &gs, int epilogue, 
 
 // CUs of the device (256 on an MI355X).
 static int device_cus() {
-    static int cus = 0;
-    if (cus == 0 && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, 0) != hipSuccess) cus = 256;
+    static const int cus = [] {  // once, also when several threads ask first
+        int n = 0;
+        return hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, 0) == hipSuccess && n > 0 ? n : 256;
+    }();
     return cus;
 }
 
