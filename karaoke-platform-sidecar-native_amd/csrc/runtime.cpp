@@ -602,15 +602,19 @@ static void launch_h2_batched(hipStream_t s, const GemmBatchH2 &b, unsigned n) {
         for (unsigned i = 0; i < n; i++) sum += tiles_of(i, bm, bn);
         return sum;
     };
-    // Problems of few columns (N < 128) are bound by reading A, not by the
-    // products the rule counts: past one tile per CU of more than half-full
-    // 256-row tiles those stay (62 bands of 801 rows, K = 1536, N 16..1032: 157 us
-    // against 190, 189, 193 on the smaller ones; 64 of 87 rows: 43, 33, 29, 27).
+    // Past one tile per CU of more than half-full 256-row tiles those stay: the
+    // rule counts products, and a batch of narrow problems (N 16..1032) is bound by
+    // reading A, a wide one (N = 1536) that fills the chip gains nothing from
+    // smaller tiles.  us on 256x128, 128x128, 64x128, 64x64: layer 1 of 62 bands
+    // (K = 384) at 87 rows 61, 44, 56, 57, at 257 119, 112, 143, 141, at 801 244,
+    // 271, 288, 312, at 3600 906, 910, 1042, 1229; layer 2 (K = 1536) at 87 81, 69,
+    // 57, 47, at 257 128, 114, 98, 102, at 801 156, 183, 185, 190.  Both layers of
+    // both models at 21 lengths from 20 to 6001: the choice within 7% of the best.
     int64_t rows = 0;
     for (unsigned i = 0; i < n; i++) rows = std::max<int64_t>(rows, b.d[i].M);
     const H2TileKind kind = rows > 128 && tiles(256, 128) > device_cus()
                                 ? H2_TILE_256
-                                : h2_tile_pick(tiles, k32, EPI == EPI_GEGLU);
+                                : h2_tile_pick(tiles, k32, false);
     with_h2_tile<EPI>(kind, [&](auto tile) {
         using T = decltype(tile);
         int64_t most = 0;
@@ -645,11 +649,8 @@ bool gemm_h2_batched(hipStream_t s, const std::vector<GemmArgsH2> &gs, const Ope
         const unsigned n = (unsigned)count;
         switch (epilogue) {
             case EPI_STORE: launch_h2_batched<EPI_STORE>(s, b, n); break;
-            case EPI_GELU: launch_h2_batched<EPI_GELU>(s, b, n); break;
             case EPI_TANH: launch_h2_batched<EPI_TANH>(s, b, n); break;
-            case EPI_RESIDUAL: launch_h2_batched<EPI_RESIDUAL>(s, b, n); break;
-            case EPI_GEGLU: launch_h2_batched<EPI_GEGLU>(s, b, n); break;
-            default: set_error("unknown GEMM epilogue %d", epilogue); return false;
+            default: set_error("gemm_h2_batched: epilogue %d is not supported", epilogue); return false;
         }
         if (!sync_debug(s, "gemm_h2_batched_kernel")) return false;
     }

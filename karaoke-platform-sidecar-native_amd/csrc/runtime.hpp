@@ -168,7 +168,8 @@ struct OperandBound {
 };
 bool gemm_h2(hipStream_t s, const GemmArgsH2 &g, const OperandBound &bound, int epilogue, KernelTimer *t = nullptr,
              const char *name = "gemm_h2");
-// A ragged batch of fp16 two-piece GEMMs with one A bound (one launch per 96 problems).
+// A ragged batch of fp16 two-piece GEMMs with one A bound (one launch per 96
+// problems), EPI_STORE or EPI_TANH.
 bool gemm_h2_batched(hipStream_t s, const std::vector<GemmArgsH2> &gs, const OperandBound &bound, int epilogue,
                      KernelTimer *t = nullptr, const char *name = "gemm_h2");
 // The mask estimator's second layer with its GLU and the reference's bin
