@@ -200,6 +200,45 @@ def test_gemm_h2_tiles_same_bits(ctx, N, K, epi):
         assert torch.equal(run(rows).view(torch.int32), whole[:rows].view(torch.int32)), rows
 
 
+def test_gemm_h2_tanh_sweep(ctx):
+    """The tanh epilogue on zero products, so on the biases alone, against float64.  Bounds in units of u = 2^-24, rounding
+    errors added at their worst: below 1 the result's rounding (u) and those of x^2, x^3 and P's Horner steps (3.2 u) on
+    x^3 P, at most 0.31 of the result, plus the fit's 4.7e-9; above, the last bits of the exponent's argument, the
+    exponential, the sum and the reciprocal (7.4 u together, exponential and reciprocal within one unit in the last
+    place) on 2 / (e + 1), at most 0.31 of the result, and the result's rounding (0.66 u).  On normal pre-activations its
+    2-norm error is below that of the fp32 GEMM's tanh."""
+    N, K, u = 1 << 20, 16, 2.0 ** -24
+    zero, w = torch.zeros(1, K, device="cuda:0"), torch.zeros(N, K, device="cuda:0")
+    planes = torch.empty(ctx.h2_bytes(N, K) // 4, device="cuda:0")
+    ctx.split_weights_h2(w, planes, N, K)
+
+    def both(x):
+        h2, fp32 = torch.empty(1, N, device="cuda:0"), torch.empty(1, N, device="cuda:0")
+        ctx.gemm_h2(zero, planes, h2, 1, N, K, bias=x, epilogue=native.EPI_TANH, a_bound=1.0)
+        ctx.gemm(zero, w, fp32, 1, N, K, bias=x, epilogue=native.EPI_TANH)
+        torch.cuda.synchronize()
+        return h2[0].double(), fp32[0].double()
+
+    for lo, hi in ((2.0 ** -20, 0.8), (0.79, 0.81), (0.8, 1.0), (0.99, 1.01), (1.0, 1.2), (1.0, 10.0)):
+        x = torch.linspace(lo, hi, N, dtype=torch.float64).float().to("cuda:0")
+        t = torch.tanh(x.double())
+        rel = ((both(x)[0] - t) / t).abs()
+        below = x < 1.0
+        assert not below.any() or rel[below].max().item() <= (1 + 3.2 * 0.31) * u + 4.7e-9, (lo, hi)
+        assert below.all() or rel[~below].max().item() <= (7.4 * 0.31 + 0.66) * u, (lo, hi)
+        assert torch.equal(both(-x)[0], -both(x)[0])
+    g = torch.Generator("cuda:0").manual_seed(3)
+    for sd in (0.39, 1.0, 3.0):
+        x = torch.randn(N, device="cuda:0", generator=g) * sd
+        h2, fp32 = both(x)
+        t = torch.tanh(x.double())
+        assert (h2 - t).norm() <= (fp32 - t).norm(), sd
+    x = torch.zeros(N, device="cuda:0")
+    x[:3] = torch.tensor([float("inf"), -float("inf"), float("nan")])
+    h2 = both(x)[0]
+    assert h2[0] == 1.0 and h2[1] == -1.0 and torch.isnan(h2[2]) and not h2[3:].any()
+
+
 def test_gemm_h2_geglu(ctx, rng):
     M, F, K = 333, 192, 384
     x = rng.standard_normal((M, K)).astype(np.float32)
