@@ -16,7 +16,7 @@ if gpu_available():
     import torch
     import oracle as O
     from vocalarc_hip import audio, native, pack
-    from vocalarc_hip.dims import CONFIG_DIMS, REFERENCE_DIMS
+    from vocalarc_hip.dims import CONFIG_DIMS, REFERENCE_DIMS, ModelDims
 
 
 @pytest.fixture(scope="module")
@@ -323,6 +323,49 @@ def test_band_split_and_mask_row_tiles(cfg2_models, ref_models, which, T, layout
     dmask = empty_dev(_to_layout(mref, layout).shape)
     dm.mask_estimate(to_dev(feats), T, dmask, layout)
     assert_close(mref, _from_layout(from_dev(dmask), layout), rtol=1e-4, atol=1e-5, min_snr=110, what="mask")
+
+
+# Shapes that neither model has: other n_fft (the workgroup-per-frame transforms), 1, 3 and 8 channels, features that
+# are no multiple of 32 or 16, a mask width that is no multiple of 32, bands of 2 to 640 inputs (some no multiple of 4
+# or 16) and more than 96 bands (three launches of the mask's second layer).
+SHAPES = {
+    "mono": dict(dim=48, n_fft=1024, hop=200, channels=1, mask_hidden=80,
+                 band_widths=(1,) * 9 + (2,) * 20 + (17, 33, 64, 50, 300)),
+    "three": dict(dim=40, n_fft=512, hop=128, channels=3, mask_hidden=48, band_widths=(1,) * 20 + (5,) * 10 + (106, 81)),
+    "eight": dict(dim=112, n_fft=128, hop=50, channels=8, mask_hidden=64, band_widths=(1,) * 25 + (40,)),
+    "many": dict(dim=64, n_fft=4096, hop=700, channels=2, mask_hidden=64, band_widths=(10,) * 151 + (11,) * 49),
+    "tiny": dict(dim=36, n_fft=2, hop=1, channels=2, mask_hidden=16, band_widths=(1, 1)),
+}
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("shape", sorted(SHAPES))
+def test_front_and_back_end_other_shapes(ctx, shape, layout):
+    d = ModelDims(depth=0, heads=1, ff_dim=64, model_frames=0, **SHAPES[shape])
+    blob = pack.synthetic_pack(d, 79)
+    om, dm = O.Model(d, blob), native.Model(ctx, d, blob)
+    rng = np.random.default_rng(len(shape))
+    length = 36 * d.hop + min(5, d.hop - 1)
+    T = d.frames(length)  # 37: a whole row tile and a ragged one
+    x = rng.standard_normal((d.channels, length)).astype(np.float32)
+    src = O.stft(d, x)
+    dsrc = empty_dev(_to_layout(src, layout).shape)
+    dm.stft(to_dev(x), length, dsrc, layout)
+    assert_close(src, _from_layout(from_dev(dsrc), layout), rtol=1e-6, atol=4e-6, min_snr=120, what="stft")
+    mask = rng.standard_normal(src.shape).astype(np.float32)
+    dout = empty_dev((d.channels, length))
+    dm.istft(to_dev(_to_layout(src, layout)), to_dev(_to_layout(mask, layout)), length, dout, layout)
+    assert_close(O.istft(d, src, mask, length), from_dev(dout), rtol=1e-5, atol=4e-6, min_snr=120, what="istft")
+    ref = om.band_split(src)
+    dout = empty_dev(ref.shape)
+    dm.band_split(to_dev(_to_layout(src, layout)), T, dout, layout)
+    assert_close(ref, from_dev(dout), rtol=1e-4, atol=2e-5, min_snr=110, what="band split")
+    feats = rng.standard_normal((T, d.bands, d.dim), dtype=np.float32)
+    ref = om.mask_estimate(feats)
+    dmask = empty_dev(_to_layout(ref, layout).shape)
+    dm.mask_estimate(to_dev(feats), T, dmask, layout)
+    assert_close(ref, _from_layout(from_dev(dmask), layout), rtol=1e-4, atol=1e-5, min_snr=110, what="mask")
+    dm.close()
 
 
 @pytest.mark.parametrize("name,power", [("weight", 121), ("weight", -110), ("gamma", 118), ("gamma", -118)])
