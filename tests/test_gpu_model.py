@@ -57,16 +57,18 @@ def test_transformer_block_config(cfg2_models, rng, axis, S, L):
     assert_close(ref, out, rtol=1e-4, atol=1e-4, min_snr=100, what="transformer (config)")
 
 
-@pytest.mark.parametrize("axis,S,L", [(0, 4, 62), (1, 3, 801), (1, 2, 97)])
+@pytest.mark.parametrize("axis,S,L", [(0, 4, 62), (1, 3, 801), (1, 2, 161)])
 def test_transformer_block_kv_prescale_bit_identical(cfg2_models, rng, monkeypatch, axis, S, L):
     """The fused block's QKV GEMM writes k and v times the attention's piece
     scales (2^ek, 2^ev: one ldexp exponent per 32-column tile) and the
     attention stages them unscaled; VOCALARC_KV_PRESCALE=0 keeps the
     unscaled projection and the scaling multiplies in the attention.  Both
     must give the same bits (powers of two commute with the rotation and the
-    splits), on both axes and on a ragged length.  The band axis runs its
-    projection and attention as the two kernels here (VOCALARC_BAND_FUSED=0:
-    the fused kernel always scales k and v in its epilogue)."""
+    splits), on both axes and on a ragged length (64 < L <= 128 never scales
+    them).  The band axis runs its projection and attention as the two kernels
+    here (VOCALARC_BAND_FUSED=0: the fused kernel always scales k and v in its
+    epilogue).  A block alone norms x as a pass; the norm inside the projection
+    is test_forward_kv_prescale_bit_identical's."""
     om, dm = cfg2_models
     x = rng.standard_normal((S, L, om.d.dim), dtype=np.float32)
     monkeypatch.setenv("VOCALARC_BAND_FUSED", "0")
@@ -84,15 +86,36 @@ def test_transformer_block_kv_prescale_bit_identical(cfg2_models, rng, monkeypat
     assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
 
 
+@pytest.mark.parametrize("pieces", [None, "0"])
+def test_forward_kv_prescale_bit_identical(cfg2_models, monkeypatch, pieces):
+    """Two layers on 201 frames: from the second block on the attention's norm runs inside the QKV GEMM, whose k and v
+    leave scaled (with VOCALARC_KV_PIECES=0 as fp32, else split) or, with VOCALARC_KV_PRESCALE=0, as they are: the same
+    bits.  The band axis on the two kernels, as above."""
+    om, dm = cfg2_models
+    x = audio.sine_mix(2.0, 16)
+    monkeypatch.setenv("VOCALARC_BAND_FUSED", "0")
+    if pieces is not None:
+        monkeypatch.setenv("VOCALARC_KV_PIECES", pieces)
+    outs = []
+    for env in (None, "0"):
+        if env is not None:
+            monkeypatch.setenv("VOCALARC_KV_PRESCALE", env)
+        dx = empty_dev(x.shape)
+        dm.forward(to_dev(x), x.shape[1], dx)
+        outs.append(from_dev(dx))
+    assert np.all(np.isfinite(outs[0]))
+    assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+
+
 @pytest.mark.parametrize("S,L", [(4, 62), (23, 62), (5, 64), (7, 17), (3, 1)])
 def test_band_attention_fused(cfg2_models, rng, monkeypatch, S, L):
     """The band axis's pre-norm projection and attention in one kernel
     (sequences of L <= 64 consecutive rows; q, k, v and the gate logits stay
     on chip), against the oracle and against the two kernels it replaces
-    (VOCALARC_BAND_FUSED=0).  q, k and v are formed by the same expressions
-    as the QKV GEMM's; the gate logit is an fp32 dot product instead of the
-    split GEMM's column, so the two paths agree to a few fp32 roundings of the
-    gate, not bit for bit.  Odd S leaves a tile with one sequence, L = 64
+    (VOCALARC_BAND_FUSED=0).  The fused kernel splits x and norms the products;
+    a block alone on the two kernels norms x as a pass and splits the normed
+    rows.  The gate logit is an fp32 dot product instead of the split GEMM's
+    column.  So the two paths agree to a few fp32 roundings, not bit for bit.  Odd S leaves a tile with one sequence, L = 64
     fills a tile's 64 positions, L = 1 is a single key."""
     om, dm = cfg2_models
     x = rng.standard_normal((S, L, om.d.dim), dtype=np.float32)
@@ -323,6 +346,34 @@ def test_band_split_and_mask_row_tiles(cfg2_models, ref_models, which, T, layout
     dmask = empty_dev(_to_layout(mref, layout).shape)
     dm.mask_estimate(to_dev(feats), T, dmask, layout)
     assert_close(mref, _from_layout(from_dev(dmask), layout), rtol=1e-4, atol=1e-5, min_snr=110, what="mask")
+
+
+@pytest.mark.parametrize("which", ["config", "reference"])
+def test_band_split_error_within_fp32_mfma(cfg2_models, ref_models, cfg2, ref_pack, which):
+    """The pieces' products against float64: no further off than the same bands on the fp32 MFMA instruction, on normal
+    spectra, on a tone mix's and on bins of very different level (the operands' 22 bits cost less than the fp32
+    accumulation's roundings saved by 16-wide products)."""
+    om, dm = cfg2_models if which == "config" else ref_models
+    d, blob = om.d, cfg2[1] if which == "config" else ref_pack
+    views, rng = pack.tensor_views(d, blob), np.random.default_rng(12)
+    normal = rng.standard_normal((d.freq_bins, d.channels, 70, 2)).astype(np.float32)
+    levels = (10.0 ** rng.uniform(-6, 0, normal.shape[:3])).astype(np.float32)[..., None]
+    for name, src in (("normal", normal), ("tones", O.stft(d, audio.sine_mix(0.8, 5))), ("levels", normal * levels)):
+        T = src.shape[2]
+        ref = np.empty((d.bands, T, d.dim))
+        for b, (f0, w) in enumerate(zip(d.first_frequencies(), d.band_widths)):
+            v = src[f0:f0 + w].astype(np.float64).transpose(2, 0, 1, 3).reshape(T, -1)
+            v *= np.sqrt(v.shape[1]) / np.sqrt((v * v).sum(1, keepdims=True) + 1e-12)
+            wm = pack.unpack_matrix(views[f"bands.{b}.weight"], d.dim, v.shape[1]).astype(np.float64)
+            ref[b] = (v * views[f"bands.{b}.gamma"]) @ wm.T + views[f"bands.{b}.bias"]
+        err = {}
+        for precision in (native.PRECISION_FP32, native.PRECISION_FP32_MFMA):
+            dm.set_precision(precision)
+            out = empty_dev(ref.shape)
+            dm.band_split(to_dev(src), T, out)
+            err[precision] = np.linalg.norm(from_dev(out) - ref) / np.linalg.norm(ref)
+        dm.set_precision(native.PRECISION_FP32)
+        assert err[native.PRECISION_FP32] <= err[native.PRECISION_FP32_MFMA], (name, err)
 
 
 # Shapes that neither model has: other n_fft (the workgroup-per-frame transforms), 1, 3 and 8 channels, features that
