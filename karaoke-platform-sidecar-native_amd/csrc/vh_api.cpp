@@ -730,7 +730,8 @@ bool prepare_split(vh_model *m) {
 
 // The band split's descriptors: weight pieces and gains padded to K chunks of
 // 16, the exponent of each band's normalised rows.
-constexpr int BAND_CLASSES = 4, BAND_CLASS_K[BAND_CLASSES] = {64, 192, 528, 640};
+constexpr int BAND_CLASSES = 4, BAND_CLASS_K[BAND_CLASSES] = {64, 192, 528, 640},
+              BAND_CLASS_ROWS[BAND_CLASSES] = {32, 64, 32, 32};  // band_split_kernel's KMAX and RT
 bool prepare_band_split(vh_model *m) {
     const Dims &d = m->d;
     hipStream_t s = m->ctx->work_stream();
@@ -867,12 +868,14 @@ bool stage_band_split(vh_model *m, const float *source, const SpecLayout &lay, i
             a.count = (int)m->band_class[c].size();
             list += a.count;
             if (!a.count) continue;
-            const int rt = c == 1 ? 64 : 32;
-            const dim3 grid((unsigned)((M + rt - 1) / rt) * (unsigned)a.count);
-            if (c == 0) hipLaunchKernelGGL((band_split_kernel<32, BAND_CLASS_K[0], 3, 256, 4>), grid, dim3(256), 0, s, a);
-            else if (c == 1) hipLaunchKernelGGL((band_split_kernel<64, BAND_CLASS_K[1], 3, 512, 12>), grid, dim3(512), 0, s, a);
-            else if (c == 2) hipLaunchKernelGGL((band_split_kernel<32, BAND_CLASS_K[2], 2, 512, 17>), grid, dim3(512), 0, s, a);
-            else hipLaunchKernelGGL((band_split_kernel<32, BAND_CLASS_K[3], 2, 512, 10>), grid, dim3(512), 0, s, a);
+            auto launch = [&](auto kernel, int threads) {
+                const unsigned tiles = (unsigned)((M + BAND_CLASS_ROWS[c] - 1) / BAND_CLASS_ROWS[c]);
+                hipLaunchKernelGGL(kernel, dim3(tiles * (unsigned)a.count), dim3(threads), 0, s, a);
+            };
+            if (c == 0) launch(band_split_kernel<BAND_CLASS_ROWS[0], BAND_CLASS_K[0], 3, 256, 4>, 256);
+            else if (c == 1) launch(band_split_kernel<BAND_CLASS_ROWS[1], BAND_CLASS_K[1], 3, 512, 12>, 512);
+            else if (c == 2) launch(band_split_kernel<BAND_CLASS_ROWS[2], BAND_CLASS_K[2], 2, 512, 17>, 512);
+            else launch(band_split_kernel<BAND_CLASS_ROWS[3], BAND_CLASS_K[3], 2, 512, 10>, 512);
             if (!sync_debug(s, "band_split_kernel")) return false;
         }
         return true;
