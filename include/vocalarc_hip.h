@@ -213,8 +213,12 @@ void vh_model_free(vh_model *model);
      at load), and so does the attention on both axes (the two-piece
      kernels of VH_ATT_H2, scaled from the fused projection's weight bound;
      a layer whose bound lies outside their scale range runs its attention
-     on the kernels without piece scales).
-   VH_PRECISION_FP32_MFMA: every product on the fp32 MFMA instruction.
+     on the kernels without piece scales; a band split whose weights or gains
+     do runs on the fp32 MFMA instruction).  An operand's two pieces hold 22 of
+     its 24 bits; the products' error against 64 bits is measured below the
+     fp32 MFMA instruction's, which rounds its sums eight times as often.
+   VH_PRECISION_FP32_MFMA: every product on the fp32 MFMA instruction, the
+     operands' 24 bits.
    VH_PRECISION_BF16: activations rounded to bf16 as they enter the matrix
      cores, bf16 weight copies made on the first switch, fp32 accumulation,
      normalisation, softmax and DSP (separately reported variant).

@@ -378,8 +378,9 @@ __global__ __launch_bounds__(64 * WAVES, 3) void attention_h2_kernel(AttnArgs a)
 // the 4 x 16 block (4 keys x 16 dims) the group addresses -- two reads per
 // piece give the 8 keys of a lane's operand in the probabilities' key order.
 // The key blocks' pipeline, softmax and output are those of
-// attention_h2_kernel (same bits); only the time axis with 32-bit staging
-// offsets takes this path (OFF32).
+// attention_h2_kernel (same bits); transformer_block takes it past 128 keys,
+// on the row orders whose positions the projection finds, with 32-bit staging
+// offsets.
 constexpr int KVP_ROW = 128;                 // bytes of one piece of one key (64 halves)
 constexpr int KVP_PIECE = ATT_KB * KVP_ROW;  // 4 KB: one piece of a 32-key block
 VH_DEVICE int kvp_swz_k(int r) { return (r >> 1) & 7; }
