@@ -45,12 +45,14 @@ typedef struct vh_model vh_model;
 vh_context *vh_create(void);
 /* Also frees every model loaded in ctx that vh_model_free has not freed. */
 void vh_destroy(vh_context *ctx);
-/* Later calls issue their work on hip_stream, after all that the context has
-   issued on its earlier streams (its scratch is shared): the new stream waits
-   for an event recorded on the old one, the host does not.  No order is made
-   into or out of a stream that is capturing; the next switch between streams
-   that are not makes it up.  A stream with work that vh_synchronize has not
-   completed may be destroyed only after the switch away from it. */
+/* Later calls issue their work on hip_stream.  The context and its models have
+   scratch that calls share.  After a change of stream the next call that uses
+   it waits, on the device, for the last vh_mask_estimate, vh_forward or
+   vh_separate, and for every call issued on the null stream (not into a capture,
+   whose work runs when the graph does).  Between other calls on other streams
+   (vh_transformer, vh_istft, vh_band_split, vh_attention with VH_ATT_H2,
+   vh_gemm_h2 without a bound), and for the caller's own buffers, the order is the
+   caller's: vh_synchronize before the change, or an event of their own. */
 int vh_set_stream(vh_context *ctx, void *hip_stream);
 int vh_synchronize(vh_context *ctx);
 const char *vh_last_error(void);

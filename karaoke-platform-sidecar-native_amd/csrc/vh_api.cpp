@@ -7,6 +7,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <optional>
 #include <vector>
 
 #include "band_split.hpp"
@@ -31,13 +32,11 @@ struct vh_model;
 
 struct vh_context {
     hipStream_t stream = nullptr;
-    bool issued = false;                 // work issued on `stream` since it was set or synchronised
-    std::vector<hipStream_t> unordered;  // earlier streams that the present one does not wait for yet (vh_set_stream)
-    hipEvent_t switched = nullptr;
-    hipStream_t work_stream() {
-        issued = true;
-        return stream;
-    }
+    // the end of the last call that left one for the next stream (SharedScratch)
+    hipEvent_t ended = nullptr;
+    bool outstanding = false;  // such a call since the last vh_synchronize
+    bool recorded = false;     // `ended` holds its end; no: it ran on the null stream
+    bool owed = false;         // the stream has changed since: the next one waits for it
     std::vector<vh_model *> models;  // live models (vh_destroy frees those left)
     int device = 0;
     char name[256] = "";
@@ -149,57 +148,63 @@ extern "C" void vh_destroy(vh_context *ctx) {
     for (vh_model *m : ctx->models) delete m;  // models not freed by their owner
     ctx->models.clear();
     ctx->timer.reset();
-    if (ctx->switched) (void)hipEventDestroy(ctx->switched);
+    if (ctx->ended) (void)hipEventDestroy(ctx->ended);
     delete ctx;
 }
 
-static bool is_capturing(hipStream_t s) {
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
+// In a call that uses the scratch of the context or of a model: no call waits
+// for its own end, so the first one after a change of stream waits, on the
+// device, for the end of the last that left one.  That end is recorded while
+// its stream is known to exist (the owner may destroy it before the change): by
+// calls that LEAVE one when they return, or for the null stream, which always
+// exists, when it is waited for.  The short calls leave none on other streams: it
+// takes 3-5 us of a 97 us block, beside 4 ms of the shortest forward and 73 us
+// of the shortest mask estimate (which took 168 while it ended in a host wait).
+// Calls into a capture neither wait nor record: their work runs when the graph
+// does.
+enum Ending { NO_END, LEAVE_END };
+struct SharedScratch {
+    vh_context *ctx;
+    const Ending ending;
+    bool captured = false, ok = true;
+    explicit SharedScratch(vh_context *c, Ending e = NO_END) : ctx(c), ending(e) {
+        if (ctx->stream && (ctx->owed || ending == LEAVE_END)) {
+            hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+            ok = check(hipStreamIsCapturing(ctx->stream, &st), "hipStreamIsCapturing");
+            captured = st != hipStreamCaptureStatusNone;
+        }
+        if (!ok || captured || !ctx->owed) return;
+        if (ctx->recorded || ctx->stream)  // else both ran on the null stream
+            ok = (ctx->recorded || record(nullptr)) &&
+                 check(hipStreamWaitEvent(ctx->stream, ctx->ended, 0), "hipStreamWaitEvent(stream order)");
+        ctx->owed = !ok;
     }
-    return st != hipStreamCaptureStatusNone;
-}
+    ~SharedScratch() {
+        if (!ok || captured || (ctx->stream && ending == NO_END)) return;
+        ctx->outstanding = true;
+        ctx->recorded = false;
+        if (ctx->stream && !record(ctx->stream)) ctx->outstanding = hipStreamSynchronize(ctx->stream) != hipSuccess;
+    }
+    bool record(hipStream_t s) {
+        if (!ctx->ended &&
+            !check(hipEventCreateWithFlags(&ctx->ended, hipEventDisableTiming), "hipEventCreate(stream order)"))
+            return false;
+        return ctx->recorded = check(hipEventRecord(ctx->ended, s), "hipEventRecord(stream order)");
+    }
+    SharedScratch(const SharedScratch &) = delete;
+};
 
-// Every call of a context shares its scratch and its models', and none waits
-// for its own end: a new stream waits for what was issued on the earlier ones.
-// Into a capture nothing can be ordered, and a capturing stream's own work runs
-// at replays, so an earlier stream is kept until a switch where neither does.
 extern "C" int vh_set_stream(vh_context *ctx, void *s) {
     if (!ctx) return 0;
-    const hipStream_t next = (hipStream_t)s;
-    if (next == ctx->stream) return 1;
-    std::vector<hipStream_t> &before = ctx->unordered;
-    if (ctx->issued && std::find(before.begin(), before.end(), ctx->stream) == before.end()) before.push_back(ctx->stream);
-    ctx->stream = next;
-    ctx->issued = false;
-    before.erase(std::remove(before.begin(), before.end(), next), before.end());  // its own order
-    if (before.empty() || is_capturing(next)) return 1;
-    if (!ctx->switched && !check(hipEventCreateWithFlags(&ctx->switched, hipEventDisableTiming), "hipEventCreate(stream)"))
-        return 0;
-    std::vector<hipStream_t> kept;
-    for (hipStream_t old : before) {
-        if (is_capturing(old)) {
-            kept.push_back(old);
-            continue;
-        }
-        if (hipEventRecord(ctx->switched, old) != hipSuccess) {  // the stream is gone: wait for its work here
-            (void)hipGetLastError();
-            if (!check(hipDeviceSynchronize(), "hipDeviceSynchronize(destroyed stream)")) return 0;
-        } else if (!check(hipStreamWaitEvent(next, ctx->switched, 0), "hipStreamWaitEvent(stream)")) {
-            return 0;
-        }
-        ctx->issued = true;  // the next switch orders after these too
-    }
-    before.swap(kept);
+    if ((hipStream_t)s != ctx->stream) ctx->owed = ctx->outstanding;
+    ctx->stream = (hipStream_t)s;
     return 1;
 }
 
 extern "C" int vh_synchronize(vh_context *ctx) {
     if (!ctx) return 0;
     bool ok = check(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
-    if (ok) ctx->issued = false;
+    if (ok && !ctx->owed) ctx->outstanding = false;
     ctx->timer.collect();
     return ok ? 1 : 0;
 }
@@ -210,23 +215,23 @@ extern "C" const char *vh_device_name(vh_context *ctx) { return ctx ? ctx->name 
 // --------------------------------------------------------- isolated kernels
 extern "C" int vh_rmsnorm(vh_context *ctx, int64_t rows, int dim, const float *x, const float *gamma, float *y) {
     if (!ctx) return 0;
-    return rmsnorm(ctx->work_stream(), x, dim, gamma, y, dim, rows, dim, &ctx->timer) ? 1 : 0;
+    return rmsnorm(ctx->stream, x, dim, gamma, y, dim, rows, dim, &ctx->timer) ? 1 : 0;
 }
 
 extern "C" int vh_rmsnorm_bf16(vh_context *ctx, int64_t rows, int dim, const float *x, const float *gamma, void *y) {
     if (!ctx) return 0;
-    return rmsnorm_bf16(ctx->work_stream(), x, dim, gamma, y, dim, rows, dim, &ctx->timer) ? 1 : 0;
+    return rmsnorm_bf16(ctx->stream, x, dim, gamma, y, dim, rows, dim, &ctx->timer) ? 1 : 0;
 }
 
 extern "C" int vh_rmsnorm_h2(vh_context *ctx, int64_t rows, int dim, const float *x, const float *gamma,
                              const float *bound, float *y) {
     if (!ctx) return 0;
-    return rmsnorm_h2(ctx->work_stream(), x, dim, gamma, y, dim, rows, dim, bound, &ctx->timer) ? 1 : 0;
+    return rmsnorm_h2(ctx->stream, x, dim, gamma, y, dim, rows, dim, bound, &ctx->timer) ? 1 : 0;
 }
 
 extern "C" int vh_softmax_rows(vh_context *ctx, int64_t rows, int len, const float *in, float *out) {
     if (!ctx) return 0;
-    return softmax_rows(ctx->work_stream(), in, out, rows, len, &ctx->timer) ? 1 : 0;
+    return softmax_rows(ctx->stream, in, out, rows, len, &ctx->timer) ? 1 : 0;
 }
 
 extern "C" int vh_rope_bhld(vh_context *ctx, int64_t bh, int len, int dim_head, float *x) {
@@ -235,24 +240,24 @@ extern "C" int vh_rope_bhld(vh_context *ctx, int64_t bh, int len, int dim_head, 
         return 0;
     }
     const float *cs, *sn;
-    if (!ctx->rope.get(len, dim_head, ctx->work_stream(), &cs, &sn)) return 0;
-    return rope_bhld(ctx->work_stream(), x, cs, sn, bh, len, &ctx->timer) ? 1 : 0;
+    if (!ctx->rope.get(len, dim_head, ctx->stream, &cs, &sn)) return 0;
+    return rope_bhld(ctx->stream, x, cs, sn, bh, len, &ctx->timer) ? 1 : 0;
 }
 
 extern "C" int vh_geglu(vh_context *ctx, int64_t rows, int width, const float *in, float *out) {
     if (!ctx) return 0;
-    return geglu(ctx->work_stream(), in, out, rows, width, &ctx->timer) ? 1 : 0;
+    return geglu(ctx->stream, in, out, rows, width, &ctx->timer) ? 1 : 0;
 }
 
 extern "C" int vh_residual_add(vh_context *ctx, int64_t n, float *x, const float *r) {
     if (!ctx) return 0;
-    return residual_add(ctx->work_stream(), x, r, n, &ctx->timer) ? 1 : 0;
+    return residual_add(ctx->stream, x, r, n, &ctx->timer) ? 1 : 0;
 }
 
 extern "C" int vh_gemm(vh_context *ctx, int64_t M, int N, int K, const float *A, int lda, const float *W, int ldw,
                        const float *bias, float *C, int ldc, int epilogue) {
     if (!ctx) return 0;
-    return gemm(ctx->work_stream(), {A, lda, W, ldw, bias, C, ldc, M, N, K}, epilogue, &ctx->timer, "gemm") ? 1 : 0;
+    return gemm(ctx->stream, {A, lda, W, ldw, bias, C, ldc, M, N, K}, epilogue, &ctx->timer, "gemm") ? 1 : 0;
 }
 
 extern "C" int vh_gemm_bf16(vh_context *ctx, int64_t M, int N, int K, const void *A, int lda, const void *Wh, int ldw,
@@ -262,14 +267,14 @@ extern "C" int vh_gemm_bf16(vh_context *ctx, int64_t M, int N, int K, const void
     g.a_bf16 = (flags & VH_BF16_A) != 0;
     g.c_bf16 = (flags & VH_BF16_C) != 0;
     g.staged = (flags & VH_BF16_STAGED) != 0;
-    return gemm_bf16(ctx->work_stream(), g, epilogue, &ctx->timer, "gemm_bf16") ? 1 : 0;
+    return gemm_bf16(ctx->stream, g, epilogue, &ctx->timer, "gemm_bf16") ? 1 : 0;
 }
 
 extern "C" int vh_gemm_split(vh_context *ctx, int64_t M, int N, int K, const float *A, int lda, const void *Ws,
                              const float *bias, float *C, int ldc, int epilogue) {
     if (!ctx) return 0;
     GemmArgsSplit g{A, lda, Ws, bias, C, ldc, M, N, K};
-    return gemm_split(ctx->work_stream(), g, epilogue, &ctx->timer, "gemm_split") ? 1 : 0;
+    return gemm_split(ctx->stream, g, epilogue, &ctx->timer, "gemm_split") ? 1 : 0;
 }
 
 extern "C" size_t vh_split_bytes(int N, int K) { return N > 0 && K > 0 ? split_bytes(N, K) : 0; }
@@ -279,12 +284,13 @@ extern "C" int vh_split_weights(vh_context *ctx, int N, int K, const float *W, i
         set_error("vh_split_weights: null argument");
         return 0;
     }
-    return split_weights(ctx->work_stream(), W, N, K, ldw_in, Ws) ? 1 : 0;
+    return split_weights(ctx->stream, W, N, K, ldw_in, Ws) ? 1 : 0;
 }
 
 extern "C" int vh_gemm_h2(vh_context *ctx, int64_t M, int N, int K, const float *A, int lda, float a_bound,
                           const void *Wp, const float *bias, float *C, int ldc, int epilogue, int flags) {
     if (!ctx || (flags & ~VH_H2_A_ROWS)) return 0;
+    std::optional<SharedScratch> scratch;
     GemmArgsH2 g{A, lda, Wp, bias, C, ldc, M, N, K};
     g.a_h2 = (flags & VH_H2_A_ROWS) != 0;
     OperandBound b{nullptr, a_bound};
@@ -294,16 +300,17 @@ extern "C" int vh_gemm_h2(vh_context *ctx, int64_t M, int N, int K, const float 
     }
     if (!(a_bound > 0.0f)) {
         // the caller gave no bound: A's own maximum
+        if (!scratch.emplace(ctx).ok) return 0;
         if (M <= 0 || K <= 0 || lda < K || !A) {
             set_error("vh_gemm_h2: bad shape M=%lld K=%d lda=%d", (long long)M, K, lda);
             return 0;
         }
         if (!ctx->bounds.ensure((64 + ABSMAX_PARTIALS) * sizeof(float), "hipMalloc(operand bound)") ||
-            !absmax(ctx->work_stream(), A, (M - 1) * lda + K, ctx->bounds.f() + 64, ctx->bounds.f()))
+            !absmax(ctx->stream, A, (M - 1) * lda + K, ctx->bounds.f() + 64, ctx->bounds.f()))
             return 0;
         b.dev = ctx->bounds.f();
     }
-    return gemm_h2(ctx->work_stream(), g, b, epilogue, &ctx->timer, "gemm_h2") ? 1 : 0;
+    return gemm_h2(ctx->stream, g, b, epilogue, &ctx->timer, "gemm_h2") ? 1 : 0;
 }
 
 extern "C" int vh_gemm_h2_ex(vh_context *ctx, int64_t M, int N, int K, const float *A, int lda,
@@ -317,7 +324,7 @@ extern "C" int vh_gemm_h2_ex(vh_context *ctx, int64_t M, int N, int K, const flo
     g.row_norm = (flags & VH_H2_ROW_NORM) != 0;
     g.zero_slot = zero_slot;
     g.amax = amax;
-    return gemm_h2(ctx->work_stream(), g, OperandBound{a_bound_dev, 0.0f}, epilogue, &ctx->timer, "gemm_h2") ? 1 : 0;
+    return gemm_h2(ctx->stream, g, OperandBound{a_bound_dev, 0.0f}, epilogue, &ctx->timer, "gemm_h2") ? 1 : 0;
 }
 
 extern "C" size_t vh_h2_bytes(int N, int K) { return N > 0 && K > 0 ? h2_bytes(N, K) : 0; }
@@ -327,38 +334,40 @@ extern "C" int vh_split_weights_h2(vh_context *ctx, int N, int K, const float *W
         set_error("vh_split_weights_h2: null argument");
         return 0;
     }
-    return split_weights_h2(ctx->work_stream(), W, N, K, ldw_in, Wp) ? 1 : 0;
+    return split_weights_h2(ctx->stream, W, N, K, ldw_in, Wp) ? 1 : 0;
 }
 
 extern "C" int vh_operand_bounds(vh_context *ctx, const float *gamma, int D, const float *W, int N, const float *b,
                                  int square, float *out) {
     if (!ctx) return 0;
-    return operand_bounds(ctx->work_stream(), gamma, D, W, N, b, square != 0, out) ? 1 : 0;
+    return operand_bounds(ctx->stream, gamma, D, W, N, b, square != 0, out) ? 1 : 0;
 }
 
 extern "C" int vh_to_bf16(vh_context *ctx, int64_t rows, int cols, const float *src, void *dst, int ld) {
     if (!ctx || rows <= 0 || cols <= 0 || ld < cols || rows * (int64_t)cols > INT32_MAX) return 0;
-    return to_bf16_rows(ctx->work_stream(), src, (int)rows, cols, dst, ld) ? 1 : 0;
+    return to_bf16_rows(ctx->stream, src, (int)rows, cols, dst, ld) ? 1 : 0;
 }
 
 extern "C" int vh_attention(vh_context *ctx, int sequences, int length, int heads, const void *qkv, void *out,
                             int apply_rotary, int flags) {
     if (!ctx || (flags & ~(VH_ATT_OUT_BF16 | VH_ATT_BF16 | VH_ATT_SPLIT | VH_ATT_H2 | VH_ATT_OUT_H2))) return 0;
+    std::optional<SharedScratch> scratch;
     const float *rt = nullptr;
-    if (apply_rotary && !ctx->rope.get_interleaved(length, 64, ctx->work_stream(), &rt)) return 0;
+    if (apply_rotary && !ctx->rope.get_interleaved(length, 64, ctx->stream, &rt)) return 0;
     const int inner = heads * 64;
     const bool h2 = (flags & VH_ATT_H2) && !(flags & VH_ATT_BF16);
     bool h2_ok = false;
     if (h2) {  // the operands' own maximum bounds them
+        if (!scratch.emplace(ctx).ok) return 0;
         if (sequences <= 0 || length <= 0 || heads <= 0 || !qkv ||
             !ctx->bounds.ensure((64 + ABSMAX_PARTIALS) * sizeof(float), "hipMalloc(operand bound)") ||
-            !absmax(ctx->work_stream(), static_cast<const float *>(qkv), (int64_t)sequences * length * 3 * inner,
+            !absmax(ctx->stream, static_cast<const float *>(qkv), (int64_t)sequences * length * 3 * inner,
                     ctx->bounds.f() + 64, ctx->bounds.f()))
             return 0;
         // outside the two-piece attention's scale range (or not finite): the
         // products run on the kernels without piece scales
         float b = 0.0f;
-        if (bounds_usable(ctx->work_stream(), ctx->bounds.f(), 1, &b) < 0) return 0;
+        if (bounds_usable(ctx->stream, ctx->bounds.f(), 1, &b) < 0) return 0;
         h2_ok = h2_attention_bound_ok(b);
     }
     const bool out_h2 = (flags & VH_ATT_OUT_H2) != 0;
@@ -366,7 +375,7 @@ extern "C" int vh_attention(vh_context *ctx, int sequences, int length, int head
         set_error("vh_attention: VH_ATT_OUT_H2 needs the two-piece kernel (VH_ATT_H2, fp32, max|qkv| in its range)");
         return 0;
     }
-    return attention(ctx->work_stream(), qkv, 3 * inner, out, inner, rt, contiguous_layout(sequences, length), heads, -1,
+    return attention(ctx->stream, qkv, 3 * inner, out, inner, rt, contiguous_layout(sequences, length), heads, -1,
                      &ctx->timer, (flags & VH_ATT_OUT_BF16) != 0, (flags & VH_ATT_BF16) != 0,
                      (flags & (VH_ATT_SPLIT | VH_ATT_H2)) != 0, h2_ok ? ctx->bounds.f() : nullptr, out_h2)
                ? 1
@@ -406,11 +415,11 @@ extern "C" int vh_attention_noalloc(vh_context *ctx, int sequences, int length, 
         // as vh_attention: the operands' own maximum bounds them (every
         // partial written before it is read); the kernels choose between the
         // two-piece products and those without piece scales on the device
-        if (!absmax(ctx->work_stream(), static_cast<const float *>(qkv), (int64_t)sequences * length * 3 * inner, scr + 64,
+        if (!absmax(ctx->stream, static_cast<const float *>(qkv), (int64_t)sequences * length * 3 * inner, scr + 64,
                     scr))
             return 0;
     }
-    return attention(ctx->work_stream(), qkv, 3 * inner, out, inner, rt, contiguous_layout(sequences, length), heads, -1,
+    return attention(ctx->stream, qkv, 3 * inner, out, inner, rt, contiguous_layout(sequences, length), heads, -1,
                      nullptr, (flags & VH_ATT_OUT_BF16) != 0, (flags & VH_ATT_BF16) != 0,
                      (flags & (VH_ATT_SPLIT | VH_ATT_H2)) != 0, h2 ? scr : nullptr, false, false, h2)
                ? 1
@@ -466,7 +475,7 @@ size_t model_weight_bytes(const Dims &d) {
 
 bool upload_pack(vh_model *m, const void *pack, size_t bytes) {
     const Dims &d = m->d;
-    hipStream_t s = m->ctx->work_stream();
+    hipStream_t s = m->ctx->stream;
     if (bytes < 64 || memcmp(pack, "VSCNAT01", 8) != 0) {
         set_error("pack: bad magic");
         return false;
@@ -611,7 +620,7 @@ bool upload_pack(vh_model *m, const void *pack, size_t bytes) {
 bool prepare_bf16(vh_model *m) {
     if (m->weights_h.ptr) return true;
     const Dims &d = m->d;
-    hipStream_t s = m->ctx->work_stream();
+    hipStream_t s = m->ctx->stream;
     const int D = d.dim, Hm = d.mask_hidden;
     auto bytes = [](int64_t rows, int cols) { return ((size_t)rows * bf16_pitch(cols) * 2 + 255) & ~(size_t)255; };
     size_t total = 0;
@@ -655,7 +664,7 @@ static float *stream_bound(vh_model *m) { return m->bounds.f() + 4 * m->layers.s
 bool prepare_split(vh_model *m) {
     if (m->weights_s.ptr) return true;
     const Dims &d = m->d;
-    hipStream_t s = m->ctx->work_stream();
+    hipStream_t s = m->ctx->stream;
     const int D = d.dim, Hm = d.mask_hidden;
     auto bytes = [](int N, int K) { return K % SPLIT_K_MULTIPLE ? 0 : (h2_bytes(N, K) + 255) & ~(size_t)255; };
     // per layer: the four matrices, and the QKV one again with its RMSNorm
@@ -734,7 +743,7 @@ constexpr int BAND_CLASSES = 4, BAND_CLASS_K[BAND_CLASSES] = {64, 192, 528, 640}
               BAND_CLASS_ROWS[BAND_CLASSES] = {32, 64, 32, 32};  // band_split_kernel's KMAX and RT
 bool prepare_band_split(vh_model *m) {
     const Dims &d = m->d;
-    hipStream_t s = m->ctx->work_stream();
+    hipStream_t s = m->ctx->stream;
     const int B = d.bands, D = d.dim;
     auto kpad = [&](int b) { return (d.in_dim(b) + GS_BK - 1) / GS_BK * GS_BK; };
     auto round = [](size_t n) { return (n + 255) & ~(size_t)255; };
@@ -811,14 +820,14 @@ bool prepare_band_split(vh_model *m) {
 // (fp32 activations; the bf16 variant rounds them as they are staged).
 bool stage_gemms(vh_model *m, const std::vector<GemmArgs> &gs, const std::vector<void *> &wh, int epi,
                  const char *name) {
-    if (m->precision != PREC_BF16) return gemm_batched(m->ctx->work_stream(), gs, epi, &m->ctx->timer, name);
+    if (m->precision != PREC_BF16) return gemm_batched(m->ctx->stream, gs, epi, &m->ctx->timer, name);
     std::vector<GemmArgsBF16> hs;
     hs.reserve(gs.size());
     for (size_t i = 0; i < gs.size(); i++) {
         const GemmArgs &g = gs[i];
         hs.push_back({g.A, g.lda, wh[i], bf16_pitch(g.K), g.bias, g.C, g.ldc, g.M, g.N, g.K});
     }
-    return gemm_bf16_batched(m->ctx->work_stream(), hs, epi, &m->ctx->timer, name);
+    return gemm_bf16_batched(m->ctx->stream, hs, epi, &m->ctx->timer, name);
 }
 
 // ---- pipeline stages on `chunks` windows at once --------------------------
@@ -836,14 +845,14 @@ bool stage_stft(vh_model *m, const float *audio, int64_t audio_len, const int64_
     a.audio = audio; a.audio_len = audio_len; a.starts = starts_dev; a.sig_len = sig_len;
     a.C = d.channels; a.T = T; a.F = d.freq_bins(); a.n_fft = d.n_fft; a.log2n = log2i(d.n_fft); a.hop = d.hop;
     a.window = m->window.f(); a.tw = static_cast<const double2_t *>(m->twiddle.ptr); a.source = source; a.out = lay;
-    Scope sc(&m->ctx->timer, m->ctx->work_stream(), "stft");
+    Scope sc(&m->ctx->timer, m->ctx->stream, "stft");
     if (d.n_fft == RF_N)
         hipLaunchKernelGGL(stft2048_kernel, dim3((T + RF_FRAMES - 1) / RF_FRAMES, chunks * d.channels),
-                           dim3(64 * RF_FRAMES), 0, m->ctx->work_stream(), a);
+                           dim3(64 * RF_FRAMES), 0, m->ctx->stream, a);
     else
-        hipLaunchKernelGGL(stft_kernel, dim3(T, chunks * d.channels), dim3(256), fft_lds_bytes(d.n_fft), m->ctx->work_stream(),
+        hipLaunchKernelGGL(stft_kernel, dim3(T, chunks * d.channels), dim3(256), fft_lds_bytes(d.n_fft), m->ctx->stream,
                            a);
-    return sync_debug(m->ctx->work_stream(), "stft_kernel");
+    return sync_debug(m->ctx->stream, "stft_kernel");
 }
 
 // source bins (layout lay) -> rows of out: band-major (time_sequences, row
@@ -851,7 +860,7 @@ bool stage_stft(vh_model *m, const float *audio, int64_t audio_len, const int64_
 bool stage_band_split(vh_model *m, const float *source, const SpecLayout &lay, int chunks, int T, float *out,
                       bool frame_major) {
     const Dims &d = m->d;
-    hipStream_t s = m->ctx->work_stream();
+    hipStream_t s = m->ctx->stream;
     const int M = chunks * T, B = d.bands, D = d.dim;
     if (m->precision == PREC_FP32 && m->band_descs.ptr) {
         BandSplitArgs a;
@@ -915,7 +924,7 @@ bool stage_band_split(vh_model *m, const float *source, const SpecLayout &lay, i
 bool stage_mask(vh_model *m, const void *normed, bool normed_bf16, int chunks, int T, float *mask,
                 const SpecLayout &lay, bool final_normed) {
     const Dims &d = m->d;
-    hipStream_t s = m->ctx->work_stream();
+    hipStream_t s = m->ctx->stream;
     const int M = chunks * T, B = d.bands, D = d.dim, Hm = d.mask_hidden;
     const bool h = m->precision == PREC_BF16;
     if (normed_bf16 && !h) {
@@ -992,7 +1001,7 @@ bool stage_mask(vh_model *m, const void *normed, bool normed_bf16, int chunks, i
 bool stage_istft(vh_model *m, const float *source, const float *mask, const SpecLayout &lay, int chunks, int T,
                  int length, float *out, int64_t pitch) {
     const Dims &d = m->d;
-    hipStream_t s = m->ctx->work_stream();
+    hipStream_t s = m->ctx->stream;
     const int sigs = chunks * d.channels;
     if (!m->frames.ensure((size_t)sigs * T * d.n_fft * sizeof(float), "hipMalloc(istft frames)")) return false;
     IstftArgs a;
@@ -1023,10 +1032,10 @@ bool stage_stack(vh_model *m, float *x, int chunks, int T) {
     xb.dev = stream_bound(m);
     xb.scratch = absmax_scratch(m);
     for (int l = 0; l < d.depth; l++) {
-        if (!transformer_block(ctx->work_stream(), d, m->layers[2 * l], x, tokens, time_axis_layout(chunks, T, d.bands),
+        if (!transformer_block(ctx->stream, d, m->layers[2 * l], x, tokens, time_axis_layout(chunks, T, d.bands),
                                ctx->scratch, ctx->rope, &ctx->timer, m->precision, &xb))
             return false;
-        if (!transformer_block(ctx->work_stream(), d, m->layers[2 * l + 1], x, tokens, band_axis_layout(chunks, T, d.bands),
+        if (!transformer_block(ctx->stream, d, m->layers[2 * l + 1], x, tokens, band_axis_layout(chunks, T, d.bands),
                                ctx->scratch, ctx->rope, &ctx->timer, m->precision, &xb))
             return false;
     }
@@ -1052,9 +1061,9 @@ bool run_windows(vh_model *m, const float *audio, int64_t audio_len, const int64
     if (!stage_band_split(m, m->source.f(), lay, chunks, T, m->x.f(), true)) return false;
     if (!stage_stack(m, m->x.f(), chunks, T)) return false;
     const bool h = m->precision == PREC_BF16;
-    if (h ? !rmsnorm_bf16(m->ctx->work_stream(), m->x.f(), d.dim, m->final_gamma, m->normed.ptr, d.dim, tokens, d.dim,
+    if (h ? !rmsnorm_bf16(m->ctx->stream, m->x.f(), d.dim, m->final_gamma, m->normed.ptr, d.dim, tokens, d.dim,
                           &m->ctx->timer)
-          : !rmsnorm(m->ctx->work_stream(), m->x.f(), d.dim, m->final_gamma, m->normed.f(), d.dim, tokens, d.dim,
+          : !rmsnorm(m->ctx->stream, m->x.f(), d.dim, m->final_gamma, m->normed.f(), d.dim, tokens, d.dim,
                      &m->ctx->timer))
         return false;
     if (!stage_mask(m, m->normed.ptr, h, chunks, T, m->mask.f(), lay, true)) return false;
@@ -1105,13 +1114,15 @@ extern "C" void vh_model_free(vh_model *m) {
 
 extern "C" int vh_transformer(vh_context *ctx, vh_model *m, int layer, int axis, float *x, int S, int L) {
     if (!ctx || !m || layer < 0 || layer >= m->d.depth || axis < 0 || axis > 1 || S <= 0 || L <= 0) return 0;
+    SharedScratch scratch(ctx);
+    if (!scratch.ok) return 0;
     // the stream's bound, for the fused band axis: found by an absmax pass
     // (float 8 of the context's bounds)
     if (!ctx->bounds.ensure((64 + ABSMAX_PARTIALS) * sizeof(float), "hipMalloc(operand bounds)")) return 0;
     XBound xb;
     xb.dev = ctx->bounds.f() + 8;
     xb.scratch = ctx->bounds.f() + 64;
-    return transformer_block(ctx->work_stream(), m->d, m->layers[2 * layer + axis], x, (int64_t)S * L, contiguous_layout(S, L),
+    return transformer_block(ctx->stream, m->d, m->layers[2 * layer + axis], x, (int64_t)S * L, contiguous_layout(S, L),
                              ctx->scratch, ctx->rope, &ctx->timer, m->precision, &xb)
                ? 1
                : 0;
@@ -1141,6 +1152,8 @@ extern "C" int vh_istft(vh_context *ctx, vh_model *m, const float *source, const
     const int T = m->d.frames(length);
     SpecLayout lay;
     if (!spec_layout_of(layout, m->d, T, &lay)) return 0;
+    SharedScratch scratch(m->ctx);
+    if (!scratch.ok) return 0;
     return stage_istft(m, source, mask, lay, 1, T, length, audio, length) ? 1 : 0;
 }
 
@@ -1149,6 +1162,8 @@ extern "C" int vh_band_split(vh_context *ctx, vh_model *m, const float *source, 
     if (!ctx || !m || frames <= 0) return 0;
     SpecLayout lay;
     if (!spec_layout_of(layout, m->d, frames, &lay)) return 0;
+    SharedScratch scratch(m->ctx);
+    if (!scratch.ok) return 0;
     return stage_band_split(m, source, lay, 1, frames, time_sequences, false) ? 1 : 0;
 }
 
@@ -1157,18 +1172,22 @@ extern "C" int vh_mask_estimate(vh_context *ctx, vh_model *m, const float *featu
     if (!ctx || !m || frames <= 0) return 0;
     SpecLayout lay;
     if (!spec_layout_of(layout, m->d, frames, &lay)) return 0;
+    SharedScratch scratch(m->ctx, LEAVE_END);
+    if (!scratch.ok) return 0;
     return stage_mask(m, features, false, 1, frames, mask, lay, false) ? 1 : 0;
 }
 
 extern "C" int vh_forward(vh_context *ctx, vh_model *m, const float *audio, int length, float *vocals,
                           float *instrumental) {
     if (!ctx || !m || length <= 0) return 0;
+    SharedScratch scratch(m->ctx, LEAVE_END);
+    if (!scratch.ok) return 0;
     if (!run_windows(m, audio, length, nullptr, length, 1, vocals, length)) return 0;
     if (instrumental) {
         const int64_t n = (int64_t)m->d.channels * length;
-        hipLaunchKernelGGL(subtract_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx->work_stream(), audio, vocals,
+        hipLaunchKernelGGL(subtract_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx->stream, audio, vocals,
                            instrumental, n);
-        if (!sync_debug(ctx->work_stream(), "subtract_kernel")) return 0;
+        if (!sync_debug(ctx->stream, "subtract_kernel")) return 0;
     }
     return 1;
 }
@@ -1180,8 +1199,10 @@ extern "C" int vh_separate(vh_context *ctx, vh_model *m, const float *audio, int
         return 0;
     }
     const Dims &d = m->d;
+    SharedScratch scratch(m->ctx, LEAVE_END);
+    if (!scratch.ok) return 0;
     const int count = length <= chunk ? 1 : 1 + (length - chunk + step - 1) / step;
-    hipStream_t s = ctx->work_stream();
+    hipStream_t s = ctx->stream;
     std::vector<int64_t> starts(count);
     for (int k = 0; k < count; k++) starts[k] = (int64_t)k * step;
     if (!m->starts.ensure(count * sizeof(int64_t), "hipMalloc(chunk starts)") ||

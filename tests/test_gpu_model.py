@@ -442,14 +442,15 @@ def test_band_split_outside_scale_range(ctx, name, power):
 
 @pytest.mark.parametrize("precision", [0, 1, 2])
 def test_stream_switch_keeps_order(ctx, cfg2_models, precision):
-    """A context's calls share its scratch, so a new stream waits for the work issued on the old one: the end of a call
-    on B implies that of a long one on A, and mask estimates issued in turn on two streams give what they give on one."""
+    """A context's calls share its scratch, so after a change of stream one waits for the last mask estimate: the end of a
+    call on B implies that of one on A behind a long product, also from and to the null stream, over a block that leaves
+    no end of its own, and mask estimates issued in turn on two streams give what they give on one."""
     om, dm = cfg2_models
     d, T = om.d, 301
     g = torch.Generator("cuda:0").manual_seed(31 + precision)
     feats = [torch.randn(T, d.bands, d.dim, device="cuda:0", generator=g) * s for s in (1.0, 3.0, 0.1, 2.0)]
     shape = (d.freq_bins, d.channels, T, 2)
-    big, small = torch.randn(8192, 8192, device="cuda:0", generator=g), torch.zeros(64, device="cuda:0")
+    big = torch.randn(8192, 8192, device="cuda:0", generator=g)
     home = torch.cuda.current_stream().cuda_stream
     a, b = torch.cuda.Stream(), torch.cuda.Stream()
     dm.set_precision(precision)
@@ -459,16 +460,22 @@ def test_stream_switch_keeps_order(ctx, cfg2_models, precision):
             want.append(empty_dev(shape))
             dm.mask_estimate(f, T, want[-1])
         torch.cuda.synchronize()
-        ctx.set_stream(a.cuda_stream)
-        with torch.cuda.stream(a):
-            for _ in range(4):
-                big @ big
-        ctx.residual_add(small, small, 32)
-        done = a.record_event()
-        ctx.set_stream(b.cuda_stream)
-        ctx.residual_add(small[32:], small[32:], 32)
-        b.synchronize()
-        assert done.query()  # B's call ended after A's
+        out, x = empty_dev(shape), torch.randn(130, d.dim, device="cuda:0", generator=g)
+        torch.cuda.synchronize()
+        for first, second in ((a, b), (torch.cuda.default_stream(), b), (a, torch.cuda.default_stream())):
+            ctx.set_stream(first.cuda_stream)
+            with torch.cuda.stream(first):
+                for _ in range(4):
+                    big @ big
+            dm.mask_estimate(feats[0], T, out)
+            done = first.record_event()
+            if first is a:
+                dm.transformer(0, 0, x, 2, 65)
+            ctx.set_stream(second.cuda_stream)
+            dm.mask_estimate(feats[0], T, out)
+            second.synchronize()
+            assert done.query()  # the second call ended after the first
+            assert torch.equal(out, want[0])
         got = [empty_dev(shape) for _ in feats]
         torch.cuda.synchronize()
         for i, (f, o) in enumerate(zip(feats, got)):
@@ -480,6 +487,28 @@ def test_stream_switch_keeps_order(ctx, cfg2_models, precision):
         dm.set_precision(native.PRECISION_FP32)
     for w, o in zip(want, got):
         assert torch.equal(w, o)
+
+
+def test_stream_destroyed_before_the_switch(ctx, cfg2_models):
+    """A stream whose work has ended may be gone when the context leaves it."""
+    import ctypes
+    om, dm = cfg2_models
+    hip = ctypes.CDLL(next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line))
+    home = torch.cuda.current_stream().cuda_stream
+    feats = torch.randn(40, om.d.bands, om.d.dim, device="cuda:0", generator=torch.Generator("cuda:0").manual_seed(7))
+    outs = [empty_dev((om.d.freq_bins, om.d.channels, 40, 2)) for _ in range(3)]
+    dm.mask_estimate(feats, 40, outs[0])
+    torch.cuda.synchronize()
+    stream = ctypes.c_void_p()
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(stream), 1) == 0
+    ctx.set_stream(stream.value)
+    dm.mask_estimate(feats, 40, outs[1])
+    torch.cuda.synchronize()  # not vh_synchronize: the context does not know
+    assert hip.hipStreamDestroy(stream) == 0
+    ctx.set_stream(home)
+    dm.mask_estimate(feats, 40, outs[2])
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
 
 
 def test_short_windows_share_row_tiles(cfg2_models):
